@@ -723,10 +723,7 @@ int hmc_chains_create(hmc_problem* hp, int64_t B, hmc_chains** out) {
       c.ex_tmp = (int32_t*)dev_alloc(c.owned, (size_t)c.B_pad * 2 * 4);
       c.ex_u = (double*)dev_alloc(c.owned, c.B_pad * 8);
       if (P.op == 1) {
-        // endpoint partial rows: residual form (n_pad / 128 row blocks), premultiplied
-        // over all of H (d_pad / 128) or over its upper block triangle (2 ceil(T/2) items)
-        const int64_t T = (P.d + 127) / 128;
-        c.n_mblocks = std::max({P.n_pad / 128, P.d_pad / 128, 2 * ((T + 1) / 2)});
+        c.n_mblocks = endpoint_max_blocks(P);
         c.partial = (double*)dev_alloc(c.owned, (size_t)c.n_mblocks * c.B_pad * 8);
         c.split_ws64_elems = gemm_split_workspace_f64(P, c.B);
         if (c.split_ws64_elems) c.split_ws64 = (double*)dev_alloc(c.owned, c.split_ws64_elems * 8);

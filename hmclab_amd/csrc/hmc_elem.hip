@@ -105,7 +105,8 @@ __device__ inline double chain_misfit(const T* x, int64_t d, const double* parti
   ob = block_sum<EW_NT>(ob, scratch);
   if (p) kk = block_sum<EW_NT>(kk, scratch);
   double lik = 0.0;
-  for (int64_t mb = 0; mb < nmb; ++mb) lik += partial[mb * ldp + c];
+  for (int64_t mb = threadIdx.x; mb < nmb; mb += EW_NT) lik += partial[mb * ldp + c];
+  lik = block_sum<EW_NT>(lik, scratch);
   double chi = 0.5 * lik + (pm + mconst);
   if (ob > 0.0) chi += INFINITY;
   if (kin) *kin = 0.5 * kk;

@@ -15,37 +15,13 @@
 // m of chain n; MFMA accumulators hold four m of one chain, so
 // the epilogue reads/writes 4-element runs of chain-major rows (bf16: 4
 // consecutive rows; f64: rows q, q+4, q+8, q+12 of a 16-row tile).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "hmc_internal.hpp"
 
 namespace hmc {
-
-// ---------------------------------------------------------------------------
-// global loads: 8 contiguous elements
-// ---------------------------------------------------------------------------
-__device__ inline void ld8(const double* p, double o[8]) {
-  const f64x2* q = reinterpret_cast<const f64x2*>(p);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f64x2 v = q[i];
-    o[2 * i] = v[0];
-    o[2 * i + 1] = v[1];
-  }
-}
-__device__ inline void ld8(const float* p, double o[8]) {
-  const floatx4* q = reinterpret_cast<const floatx4*>(p);
-  const floatx4 a = q[0], b = q[1];
-  o[0] = a[0]; o[1] = a[1]; o[2] = a[2]; o[3] = a[3];
-  o[4] = b[0]; o[5] = b[1]; o[6] = b[2]; o[7] = b[3];
-}
-__device__ inline void ld8(const uint16_t* p, double o[8]) {
-  const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-  uint32_t w[4] = {v[0], v[1], v[2], v[3]};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    o[2 * i] = bf16_bits_to_f32((uint16_t)(w[i] & 0xffffu));
-    o[2 * i + 1] = bf16_bits_to_f32((uint16_t)(w[i] >> 16));
-  }
-}
 
 // XCD-aware tile order: consecutive workgroup ids are dealt round-robin to
 // the 8 XCDs; give each XCD a contiguous range of tiles (m-major) so tiles
@@ -149,17 +125,160 @@ __device__ inline bool split_job(int gm, int gn, int nk, int F, int SPL, int& tm
 // k-tile 16, wave tile WM x WN.  K is permuted inside a k-tile: lane group
 // q at MFMA step s uses k = 4q + s, so each lane reads 4 contiguous doubles.
 // Requires A rows up to the tile edge and K padded to 16 (zeros).
+//
+// What bounds it: the matrix cores (one 16x16x4 FP64 MFMA takes a SIMD about
+// 64 clocks, so LDS and L2 are far from their limits).  Two waves per SIMD
+// with 64 accumulator registers each keep the accumulators in plain VGPRs: at
+// 128 per wave the compiler moved all of them to the accumulation registers
+// and back in every k-tile.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int WM, int WN, typename TA, typename TB, class Epi>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm_f64(
+__device__ inline void ld4(const double* p, double o[4]) {
+  const f64x2* q = reinterpret_cast<const f64x2*>(p);
+  const f64x2 a = q[0], b = q[1];
+  o[0] = a[0]; o[1] = a[1]; o[2] = b[0]; o[3] = b[1];
+}
+__device__ inline void ld4(const float* p, double o[4]) {
+  const floatx4 a = *reinterpret_cast<const floatx4*>(p);
+  o[0] = a[0]; o[1] = a[1]; o[2] = a[2]; o[3] = a[3];
+}
+__device__ inline void ld4(const uint16_t* p, double o[4]) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  o[0] = bf16_bits_to_f32((uint16_t)(v.x & 0xffffu));
+  o[1] = bf16_bits_to_f32((uint16_t)(v.x >> 16));
+  o[2] = bf16_bits_to_f32((uint16_t)(v.y & 0xffffu));
+  o[3] = bf16_bits_to_f32((uint16_t)(v.y >> 16));
+}
+
+// The k loop of one block tile, shared by the GEMM and the quadratic form.
+// Two LDS buffers, one barrier per k-tile: while the MFMAs of k-tile kt run,
+// kt + 1 is written to the other buffer and kt + 3 is on its way to registers
+// (two register sets in turn; loads past the end repeat the last tile, so the
+// counts of outstanding loads are fixed and the wait before a write leaves the
+// newer set in flight).  Keeping the MFMAs of a k-tile together, before the
+// barrier, took 8192 x 512 x 8192 from 1.06 to 0.96 ms (71 TFLOP/s); a third
+// buffer for reading fragments ahead of the barrier halves the co-resident
+// blocks and took 1.10 ms.  Rows are padded to BK + 2 doubles (conflict-free
+// fragment reads).
+template <int BM_, int BN_, int WM_, int WN_, int BK_, typename TA, typename TB>
+struct F64Tile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_, LDS = BK + 2;
+  static constexpr int CPR = BK / 4;                      // 4-element chunks per row of a k-tile
+  static constexpr int NT = (BM / WM) * (BN / WN) * 64;
+  static constexpr int TM = WM / 16, TN = WN / 16;
+  static constexpr int WPR = BN / WN;                     // waves per row of waves
+  static constexpr int BUF = (BM + BN) * LDS;          // doubles of one buffer
+  static constexpr int A_CH = (BM * CPR + NT - 1) / NT;   // chunks per thread
+  static constexpr int B_CH = (BN * CPR + NT - 1) / NT;
+
+  // acc = A[rows of the tile][k-tiles kt0..kt1) . Bt[rows of the tile][same k]^T
+  __device__ static __forceinline__ void run(const TA* __restrict__ A, int64_t lda, const TB* __restrict__ Bt,
+                                             int64_t ldb, int kt0, int kt1, double* __restrict__ smem,
+                                             doublex4 (&acc)[TM][TN]) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wm = w / WPR, wn = w % WPR;
+    const int q = lane >> 4, r = lane & 15;
+    double ra[2][A_CH][4], rb[2][B_CH][4];
+    double af[TM][4], bf[TN][4];
+    auto gload = [&](int kt, int set) {
+#pragma unroll
+      for (int i = 0; i < A_CH; ++i) {
+        const int c = tid + i * NT;
+        if ((BM * CPR) % NT == 0 || c < BM * CPR)
+          ld4(A + (int64_t)(c / CPR) * lda + (int64_t)(kt0 + kt) * BK + (c % CPR) * 4, ra[set][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < B_CH; ++i) {
+        const int c = tid + i * NT;
+        if ((BN * CPR) % NT == 0 || c < BN * CPR)
+          ld4(Bt + (int64_t)(c / CPR) * ldb + (int64_t)(kt0 + kt) * BK + (c % CPR) * 4, rb[set][i]);
+      }
+    };
+    auto put4 = [&](double* d4, const double (&v)[4]) {
+      f64x2* d = reinterpret_cast<f64x2*>(d4);
+      d[0] = f64x2{v[0], v[1]};
+      d[1] = f64x2{v[2], v[3]};
+    };
+    auto sstore = [&](double* buf, int set) {
+#pragma unroll
+      for (int i = 0; i < A_CH; ++i) {
+        const int c = tid + i * NT;
+        if ((BM * CPR) % NT == 0 || c < BM * CPR) put4(&buf[(c / CPR) * LDS + (c % CPR) * 4], ra[set][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < B_CH; ++i) {
+        const int c = tid + i * NT;
+        if ((BN * CPR) % NT == 0 || c < BN * CPR) put4(&buf[(BM + c / CPR) * LDS + (c % CPR) * 4], rb[set][i]);
+      }
+    };
+    auto get4 = [&](const double* s4, double (&v)[4]) {
+      const f64x2* sp = reinterpret_cast<const f64x2*>(s4);
+      const f64x2 u = sp[0], t = sp[1];
+      v[0] = u[0]; v[1] = u[1]; v[2] = t[0]; v[3] = t[1];
+    };
+    auto frags = [&](const double* buf, int k16) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) get4(&buf[(wm * WM + i * 16 + r) * LDS + k16 + 4 * q], af[i]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) get4(&buf[(BM + wn * WN + j * 16 + r) * LDS + k16 + 4 * q], bf[j]);
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
+
+    const int nk = kt1 - kt0;
+    if (nk <= 0) return;
+    auto upto_last = [&](int kt) { return kt < nk ? kt : nk - 1; };
+    gload(0, 0);
+    gload(upto_last(1), 1);
+    __syncthreads();   // the buffers may still be read by an earlier use
+    sstore(smem, 0);
+    gload(upto_last(2), 0);
+    __syncthreads();
+    // k-tile kt, in buffer p = kt mod 2; kt + 1 is in register set 1 - p
+    auto tile = [&](int kt, auto parity) {
+      constexpr int p = decltype(parity)::value;
+      const double* cur = smem + p * BUF;
+      frags(cur, 0);
+      sstore(smem + (1 - p) * BUF, 1 - p);
+      gload(upto_last(kt + 3), 1 - p);
+#pragma unroll
+      for (int k16 = 0; k16 < BK; k16 += 16) {
+        if (k16 > 0) frags(cur, k16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][s], bf[j][s], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+    };
+    int kt = 0;
+    for (; kt + 2 <= nk; kt += 2) {
+      tile(kt, std::integral_constant<int, 0>{});
+      tile(kt + 1, std::integral_constant<int, 1>{});
+    }
+    if (kt < nk) tile(kt, std::integral_constant<int, 0>{});
+  }
+};
+
+// waves per SIMD the register budget is set for (two for the 8-wave blocks
+// and for two co-resident 4-wave blocks)
+template <int BM, int BN, int WM, int WN, int BK, typename TA, typename TB, class Epi>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void k_gemm_f64(
     const TA* __restrict__ A, int64_t lda, const TB* __restrict__ Bt, int64_t ldb, int M, int N,
     int K, int F, int SPL, double* __restrict__ part, int64_t TR, Epi epi) {
-  constexpr int BK = 16, LDS = BK + 2;
-  constexpr int NT = (BM / WM) * (BN / WN) * 64;
-  constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int WPR = BN / WN;  // waves per row of waves
-  __shared__ double As[BM * LDS];
-  __shared__ double Bs[BN * LDS];
+  using Tile = F64Tile<BM, BN, WM, WN, BK, TA, TB>;
+  constexpr int NT = Tile::NT, TM = Tile::TM, TN = Tile::TN, WPR = Tile::WPR;
+  // the k buffers, reused by the epilogue for EN chains of the tile C[n][m]
+  constexpr int CLD = BM + 2;
+  constexpr int EN = BN > 64 ? 64 : BN;
+  constexpr int SMEM = 2 * Tile::BUF > EN * CLD ? 2 * Tile::BUF : EN * CLD;
+  __shared__ __attribute__((aligned(16))) double smem[SMEM];
 
   const int gm = (M + BM - 1) / BM, gn = (N + BN - 1) / BN;
   int tm, tn, kt0 = 0, kt1 = (K + BK - 1) / BK, sp = -1;
@@ -169,138 +288,81 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm_f64(
     return;
   }
   const int64_t m_blk = (int64_t)tm * BM, n_blk = (int64_t)tn * BN;
-  A += (int64_t)kt0 * BK;
-  Bt += (int64_t)kt0 * BK;
-
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WPR, wn = w % WPR;
   const int q = lane >> 4, r = lane & 15;
 
-  // global -> LDS mapping: rows x 16 cols in chunks of 8 elements
-  constexpr int A_CH = BM * 2 / NT;  // chunks per thread (A)
-  constexpr int B_CH = BN * 2 / NT;
-  static_assert(A_CH >= 1 && B_CH >= 1, "tile too small for thread count");
-
-  double ra[A_CH][8], rb[B_CH][8];
-  auto gload = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + i * NT, row = c >> 1, col = (c & 1) * 8;
-      ld8(A + (m_blk + row) * lda + (int64_t)kt * BK + col, ra[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < B_CH; ++i) {
-      const int c = tid + i * NT, row = c >> 1, col = (c & 1) * 8;
-      ld8(Bt + (n_blk + row) * ldb + (int64_t)kt * BK + col, rb[i]);
-    }
-  };
-  auto sstore = [&]() {
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + i * NT, row = c >> 1, col = (c & 1) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) As[row * LDS + col + e] = ra[i][e];
-    }
-#pragma unroll
-    for (int i = 0; i < B_CH; ++i) {
-      const int c = tid + i * NT, row = c >> 1, col = (c & 1) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) Bs[row * LDS + col + e] = rb[i][e];
-    }
-  };
-
   doublex4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
-
-  const int nk = kt1 - kt0;
-  gload(0);
-  for (int kt = 0; kt < nk; ++kt) {
-    __syncthreads();
-    sstore();
-    __syncthreads();
-    if (kt + 1 < nk) gload(kt + 1);
-    double af[TM][4], bfr[TN][4];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const double* src = &As[(wm * WM + i * 16 + r) * LDS + 4 * q];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) af[i][s] = src[s];
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const double* src = &Bs[(wn * WN + j * 16 + r) * LDS + 4 * q];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) bfr[j][s] = src[s];
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][s], bfr[j][s], acc[i][j], 0, 0, 0);
-  }
+  Tile::run(A + m_blk * lda, lda, Bt + n_blk * ldb, ldb, kt0, kt1, smem, acc);
 
   // D layout (measured on gfx950): lane (q, r) holds rows q, q+4, q+8, q+12 of
   // column r of each 16x16 tile
-  if (sp >= 0) {
-    // partial tile of k-range sp: part[sp][chain][row - first tail row]
-    const int64_t mt0 = (int64_t)(F / gn) * BM;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
+  if constexpr (Epi::kReduce) {
+    if (sp < 0) {
+      // per-column sums over the block's rows, deterministic order
+      __syncthreads();
+      double* red = smem;   // [BM / WM][4][BN]
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int64_t m0 = m_blk + wm * WM + i * 16 + q;
+        double colsum = 0.0;
         const int64_t n = n_blk + wn * WN + j * 16 + r;
-        if (n >= N) continue;
-        double* dst = part + ((int64_t)sp * N + n) * TR + (m0 - mt0);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dst[4 * v] = acc[i][j][v];
+        for (int i = 0; i < TM; ++i) {
+          const int64_t m0 = m_blk + wm * WM + i * 16 + q;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) colsum += epi.term(m0 + 4 * v, n, acc[i][j][v]);
+        }
+        red[(wm * 4 + q) * BN + wn * WN + j * 16 + r] = colsum;
       }
-    return;
+      __syncthreads();
+      for (int col = tid; col < BN; col += NT) {
+        double sum = 0.0;
+#pragma unroll
+        for (int a = 0; a < (BM / WM) * 4; ++a) sum += red[a * BN + col];
+        epi.store_partial(tm, n_blk + col, sum);
+      }
+      return;
+    }
   }
-  if constexpr (Epi::kReduce) {
-    // per-column sums over the block's rows, deterministic order
-    __shared__ double red[(BM / WM)][4][BN];
-    double colsum[TN];
+  // Through LDS, EN chains at a time, so that each thread handles 4
+  // consecutive rows of one chain (contiguous accesses of the chain-major
+  // arrays, one small epilogue loop): the epilogue, or the partial tile of
+  // k-range sp, part[sp][chain][row - first tail row].
+  const int64_t mt0 = (int64_t)(F / gn) * BM;
+#pragma unroll 1
+  for (int n0 = 0; n0 < BN; n0 += EN) {
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      colsum[j] = 0.0;
-      const int64_t n = n_blk + wn * WN + j * 16 + r;
+      const int nl = wn * WN + j * 16 + r - n0;
+      if (nl >= 0 && nl < EN) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int64_t m0 = m_blk + wm * WM + i * 16 + q;
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) colsum[j] += epi.term(m0 + 4 * v, n, acc[i][j][v]);
+          for (int v = 0; v < 4; ++v) smem[nl * CLD + wm * WM + i * 16 + q + 4 * v] = acc[i][j][v];
       }
-      red[wm][q][wn * WN + j * 16 + r] = colsum[j];
     }
     __syncthreads();
-    for (int col = tid; col < BN; col += NT) {
-      double s = 0.0;
-#pragma unroll
-      for (int a = 0; a < BM / WM; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) s += red[a][b][col];
-      epi.store_partial(tm, n_blk + col, s);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t m0 = m_blk + wm * WM + i * 16 + q;
-        const int64_t n = n_blk + wn * WN + j * 16 + r;
-        double v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-        epi.apply(m0, 4, n, v);
+#pragma unroll 1
+    for (int idx = tid; idx < EN * (BM / 4); idx += NT) {
+      const int nl = idx / (BM / 4), ml = 4 * (idx % (BM / 4));
+      const int64_t n = n_blk + n0 + nl;
+      const f64x2* src = reinterpret_cast<const f64x2*>(&smem[nl * CLD + ml]);
+      const f64x2 u = src[0], t = src[1];
+      if (sp >= 0) {
+        if (n >= N) continue;
+        f64x2* dst = reinterpret_cast<f64x2*>(&part[((int64_t)sp * N + n) * TR + (m_blk - mt0) + ml]);
+        dst[0] = u;
+        dst[1] = t;
+      } else if constexpr (!Epi::kReduce) {
+        const double v[4] = {u[0], u[1], t[0], t[1]};
+        epi.apply(m_blk + ml, 1, n, v);
       }
+    }
   }
 }
 
-// Split-tail epilogues of the FP64 GEMM.  Element-wise epilogues: sum the
+// Epilogues of FP64 GEMMs split along K.  Element-wise epilogues: sum the
 // SPL partials of 4 consecutive rows of one chain in fixed order, then apply.
 template <class Epi>
 __global__ __launch_bounds__(256) void k_split_epilogue_f64(const double* __restrict__ part, int SPL, int64_t TR,
@@ -706,6 +768,7 @@ struct EpiLeap {
   const double* bias;   // premultiplied FP64 trajectories: g = acc - bias[j] (or null)
   const float* gscale;  // surrogate: g = gscale[j] * acc (or null)
   const float* xsinv;   // planes hold (x - xa) * xsinv (surrogate's normalised input) (or null)
+  const T* xin = nullptr;   // positions before the stage where they are another buffer than x
   __device__ __forceinline__ void step(int64_t j, T& xv, T& pv, T g, T kk, T dd, T dd2) const {
     g += prior_grad<T>(md, j, xv);
     if (out_of_bounds(md, j, (double)xv)) g = (T)INFINITY;
@@ -763,7 +826,7 @@ struct EpiLeap {
       const int64_t j = m0 + (int64_t)k * ms;
       if (j >= M) return;
       const int64_t o = n * ld + j;
-      T xv = x[o], pv = p[o];
+      T xv = xin ? xin[o] : x[o], pv = p[o];
       T g = (T)v[k];
       if (gscale) g = (T)((float)v[k] * gscale[j]);
       if (yref) g = (T)((float)v[k] + yref[j]);
@@ -925,191 +988,225 @@ struct EpiQuad {
 // ---------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------
-// FP64 tiles: 128 x 128, 4 waves of 64 x 64.
-constexpr int F64_BM = 128, F64_BN = 128, F64_WM = 64, F64_WN = 64;
+// FP64 tiles, all of 4 waves (one per SIMD, several blocks per CU, whose
+// barriers do not line up).  128 x 64 is the fastest where its tiles give every
+// CU two blocks: 8192 x 512 x 8192 takes 0.96 ms (71 TFLOP/s) against 1.05 ms
+// with 64 x 64 and 1.50 ms with the former 128 x 128 tile of four waves.
+// Smaller tiles shorten each block's chain of k steps where there are few
+// tiles; 64 x 16 is for at most 16 chains.  128 x 128 (8 waves) keeps a
+// reducing epilogue's partial rows few.
+enum F64Cfg { F64_128x64 = 0, F64_64x64, F64_64x32, F64_32x32, F64_64x16, F64_128x128 };
+static int f64_bm(int cfg) { return cfg == F64_32x32 ? 32 : (cfg == F64_128x128 || cfg == F64_128x64) ? 128 : 64; }
+static int f64_bn(int cfg) {
+  return (cfg == F64_64x64 || cfg == F64_128x64) ? 64 : cfg == F64_64x16 ? 16 : cfg == F64_128x128 ? 128 : 32;
+}
+constexpr int F64_MAX_BN = 128;   // chain rows a tile may read past the last chain (B_pad)
+
+// Plan of one FP64 GEMM: tile and k pieces per tile (every tile is cut alike).
+// Estimated time in us: the busiest CU runs g = ceil(blocks / n_cu) blocks; a
+// 16-deep k step of them takes `lat` while one block cannot use the CU fully
+// (one wave per SIMD waits for its loads and barriers) and g * `thr` when the
+// matrix cores are busy.  A split adds its partial planes' traffic and a
+// second launch.  lat and thr are fits to measured times of 6 shapes from
+// 901 x 100 x 1536 to 8192 x 512 x 8192 in 1, 2 and 4 pieces, which the
+// estimate meets within about 10%.  Both sides of some lines: 901 x 100 x 1536
+// 16 us with 32 x 32 tiles in 4 pieces, 17 us with 64 x 32 in 4, 66 us with
+// 64 x 64 in one; 4096 x 512 x 4096 259 us with 64 x 64, 266 us with 128 x 64
+// in 2 pieces, 336 us in one.
+struct F64Plan {
+  int cfg = F64_64x64, SPL = 1;
+  int64_t TR = 0;   // rows of a partial plane: all tile rows, rounded up to 128
+  double us = 0.0;
+};
+
+constexpr double F64_MAX_WS = 256.0 * 1024 * 1024;   // bytes of partial planes
+
+static F64Plan plan_f64(int M, int N, int K, int n_cu, bool allow_split) {
+  struct Shape {
+    int cfg;
+    double lat, thr;
+  };
+  static const Shape shapes[] = {{F64_128x64, 1.25, 0.935},
+                                 {F64_64x64, 0.66, 0.49},
+                                 {F64_64x32, 0.39, 0.268},
+                                 {F64_32x32, 0.20, 0.155},
+                                 {F64_64x16, 0.25, 0.25}};
+  if (n_cu <= 0) n_cu = 256;
+  F64Plan best;
+  best.us = 1e30;
+  for (const Shape& sh : shapes) {
+    const int bm = f64_bm(sh.cfg), bn = f64_bn(sh.cfg);
+    if (sh.cfg == F64_64x16 && N > 16) continue;
+    const int64_t gm = (M + bm - 1) / bm, gn = (N + bn - 1) / bn, T = gm * gn;
+    const int64_t TR = round_up(gm * bm, 128);
+    for (int spl : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (spl > 1 && (!allow_split || K / 64 < spl)) break;
+      const double ws = 8.0 * spl * N * (double)TR;
+      if (spl > 1 && ws > F64_MAX_WS) break;
+      const double g = std::ceil((double)(T * spl) / n_cu);
+      double us = std::ceil((double)K / 16 / spl) * std::max(sh.lat, g * sh.thr);
+      if (spl > 1) us += 4.0 + 2.0 * ws / 4e6;
+      if (us < best.us) best = F64Plan{sh.cfg, spl, TR, us};
+    }
+  }
+  return best;
+}
+static size_t f64_ws_elems(const F64Plan& pl, int N) { return pl.SPL > 1 ? (size_t)pl.SPL * N * pl.TR : 0; }
+
 // BF16 tiles: 128 x 128 with a 3-stage LDS ring (144 KB); config 0 = 4 waves
 // of 64 x 64, config 1 = 8 waves of 64 x 32 (two waves per SIMD).
 constexpr int BF_BM = 128, BF_BN = 128, BF_STAGES = 3;
 
-template <typename TA, typename TB, class Epi>
-static void launch_f64(const Chains& c, const TA* A, int64_t lda, const TB* Bt, int64_t ldb, int M,
-                       int N, int K, const Epi& epi) {
-  const Problem& p = *c.p;
-  const hipStream_t s = p.stream;
-  constexpr int NT = (F64_BM / F64_WM) * (F64_BN / F64_WN) * 64;
-  const bool ws = p.split_tail && c.split_ws64;
-  SplitPlan pl = plan_split(F64_BM, F64_BN, M, N, K, p.n_cu, ws, 16);
-  if (pl.split() && (size_t)pl.SPL * N * pl.TR > c.split_ws64_elems) pl = plan_split(F64_BM, F64_BN, M, N, K, 0, false);
-  hipLaunchKernelGGL((k_gemm_f64<F64_BM, F64_BN, F64_WM, F64_WN, TA, TB, Epi>), dim3(pl.grid), dim3(NT), 0, s, A,
-                     lda, Bt, ldb, M, N, K, pl.F, pl.SPL, c.split_ws64, pl.TR, epi);
+template <int BM, int BN, int WM, int WN, int BK, typename TA, typename TB, class Epi>
+static void launch_f64_cfg(const Chains& c, const F64Plan& pl, const TA* A, int64_t lda, const TB* Bt, int64_t ldb,
+                           int M, int N, int K, const Epi& epi) {
+  constexpr int NT = (BM / WM) * (BN / WN) * 64;
+  const int gm = (M + BM - 1) / BM, gn = (N + BN - 1) / BN;
+  const int F = pl.SPL > 1 ? 0 : gm * gn;
+  const int grid = pl.SPL > 1 ? (gm * gn * pl.SPL + 7) / 8 * 8 : grid_for(gm, gn);
+  hipLaunchKernelGGL((k_gemm_f64<BM, BN, WM, WN, BK, TA, TB, Epi>), dim3(grid), dim3(NT), 0, c.p->stream, A, lda, Bt,
+                     ldb, M, N, K, F, pl.SPL, c.split_ws64, pl.TR, epi);
   HMC_HIP(hipGetLastError());
-  if (pl.split()) {
+}
+
+template <typename TA, typename TB, class Epi>
+static void launch_f64(const Chains& c, const F64Plan& pl, const TA* A, int64_t lda, const TB* Bt, int64_t ldb, int M,
+                       int N, int K, const Epi& epi) {
+  const hipStream_t s = c.p->stream;
+  switch (pl.cfg) {
+    case F64_128x64: launch_f64_cfg<128, 64, 64, 32, 16>(c, pl, A, lda, Bt, ldb, M, N, K, epi); break;
+    case F64_64x64: launch_f64_cfg<64, 64, 32, 32, 16>(c, pl, A, lda, Bt, ldb, M, N, K, epi); break;
+    case F64_64x32: launch_f64_cfg<64, 32, 32, 16, 16>(c, pl, A, lda, Bt, ldb, M, N, K, epi); break;
+    case F64_32x32: launch_f64_cfg<32, 32, 16, 16, 32>(c, pl, A, lda, Bt, ldb, M, N, K, epi); break;
+    case F64_64x16: launch_f64_cfg<64, 16, 16, 16, 32>(c, pl, A, lda, Bt, ldb, M, N, K, epi); break;
+    default:
+      if constexpr (Epi::kReduce) launch_f64_cfg<128, 128, 64, 32, 16>(c, pl, A, lda, Bt, ldb, M, N, K, epi);
+      else throw Error{HMC_ERR_STATE, "FP64 GEMM tile"};
+  }
+  if (pl.SPL > 1) {
     if constexpr (Epi::kReduce) {
       hipLaunchKernelGGL((k_split_reduce_f64<Epi>), dim3((N + 3) / 4, (unsigned)(pl.TR / 128)), dim3(256), 0, s,
-                         c.split_ws64, pl.SPL, pl.TR, N, pl.mt0, epi);
+                         c.split_ws64, pl.SPL, pl.TR, N, (int64_t)0, epi);
     } else {
       const int64_t work = (int64_t)N * (pl.TR / 4);
       const int blocks = (int)std::min<int64_t>((work + 255) / 256, 4096);
       hipLaunchKernelGGL((k_split_epilogue_f64<Epi>), dim3(blocks), dim3(256), 0, s, c.split_ws64, pl.SPL, pl.TR, N,
-                         pl.mt0, epi);
+                         (int64_t)0, epi);
     }
     HMC_HIP(hipGetLastError());
   }
 }
 
+// plan for this chain set's workspace
+static F64Plan chains_plan_f64(const Chains& c, int M, int N, int K) {
+  F64Plan pl = plan_f64(M, N, K, c.p->n_cu, c.p->split_tail && c.split_ws64);
+  if (f64_ws_elems(pl, N) > c.split_ws64_elems) pl = plan_f64(M, N, K, c.p->n_cu, false);
+  return pl;
+}
+
+template <typename TA, typename TB, class Epi>
+static void launch_f64(const Chains& c, const TA* A, int64_t lda, const TB* Bt, int64_t ldb, int M, int N, int K,
+                       const Epi& epi) {
+  launch_f64(c, chains_plan_f64(c, M, N, K), A, lda, Bt, ldb, M, N, K, epi);
+}
+
 // ---------------------------------------------------------------------------
 // Premultiplied endpoint over the upper block triangle of the symmetric H, in
-// 128-row blocks a (T of them):
+// 64-row blocks a (T of them):
 //   x^T H x - 2 b^T x = sum_a [ x_a^T H_aa x_a - 2 b_a^T x_a + 2 sum_{c>a} x_a^T H_ac x_c ],
 // half the FP64 MFMA work of the full product.  Row blocks a and T-1-a are
 // paired (T + 1 k-blocks of work per pair) and each pair's concatenated
-// k-block list is cut into two halves, so the 2 ceil(T/2) items per chain
-// tile carry equal work.  An item's rows are reduced against x right after
-// each k-range (weight 1 on the diagonal block, which also takes the b term,
-// 2 beyond it), and item i writes partial[i][chain]; the sum over items is
-// the quadratic form.  The k loop is the one of k_gemm_f64.
+// k-block list is cut into `parts` equal pieces, so the parts * ceil(T/2)
+// items per chain tile carry equal work.  An item's rows are reduced against x
+// right after each k-range (weight 1 on the diagonal block, which also takes
+// the b term, 2 beyond it), and item i writes partial[i][chain]; the sum over
+// items is the quadratic form.  The k loop is the one of k_gemm_f64, and so is
+// what bounds it (the FP64 matrix cores): 8192 parameters, 512 chains take
+// 0.89 ms with 128-row blocks of four waves, one per CU, 0.84 ms with these,
+// four per CU, and 0.62 ms (55 TFLOP/s) with each XCD on a range of items.
 // ---------------------------------------------------------------------------
-template <typename TB>
-__global__ __launch_bounds__((F64_BM / F64_WM) * (F64_BN / F64_WN) * 64) void k_quad_sym(
+constexpr int QS_BM = 64, QS_PARTS = 8;   // rows of a block, most pieces of a pair
+
+template <int BN, int WM, int WN, int BK, typename TB>
+__global__ __launch_bounds__((QS_BM / WM) * (BN / WN) * 64, 2) void k_quad_sym(
     const double* __restrict__ H, int64_t ldh, const TB* __restrict__ X, int64_t ldx,
-    const double* __restrict__ hb, int d, int N, double* __restrict__ partial, int64_t ldp) {
-  constexpr int BM = F64_BM, BN = F64_BN, WM = F64_WM, WN = F64_WN, BK = 16, LDS = BK + 2;
-  constexpr int NT = (BM / WM) * (BN / WN) * 64;
-  constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int WPR = BN / WN;
-  constexpr int KB = BM / BK;   // k steps per 128-wide k block
-  constexpr int A_CH = BM * 2 / NT, B_CH = BN * 2 / NT;
-  __shared__ double As[BM * LDS];
-  __shared__ double Bs[BN * LDS];
-  __shared__ double red[BM / WM][4][BN];
+    const double* __restrict__ hb, int d, int N, int parts, double* __restrict__ partial, int64_t ldp) {
+  constexpr int BM = QS_BM;
+  using Tile = F64Tile<BM, BN, WM, WN, BK, double, TB>;
+  constexpr int NT = Tile::NT, TM = Tile::TM, TN = Tile::TN, WPR = Tile::WPR;
+  constexpr int KB = BM / BK;   // k steps per k block
+  __shared__ __attribute__((aligned(16))) double smem[2 * Tile::BUF];
+  static_assert((BM / WM) * 4 * BN <= 2 * Tile::BUF, "reduction buffer");
 
   const int T = (d + BM - 1) / BM;
-  const int KT = (int)(ldh / BK);   // k steps of a row of H (ldh is a multiple of 16)
-  const int pr = (int)blockIdx.x >> 1, half = (int)blockIdx.x & 1;
-  const int64_t n_blk = (int64_t)blockIdx.y * BN;
+  const int KT = (int)(ldh / BK);   // k steps of a row of H (ldh is a multiple of 64)
+  // items dealt to the XCDs in contiguous ranges, an item's chain tiles
+  // together: neighbouring pairs walk neighbouring k blocks of the same chains,
+  // and the chain tiles of an item read the same rows of H
+  int item, ny;
+  if (!map_tile((T + 1) / 2 * parts, (N + BN - 1) / BN, item, ny)) return;
+  const int pr = item / parts, part = item % parts;
+  const int64_t n_blk = (int64_t)ny * BN;
   const int a1 = pr, a2 = T - 1 - pr;   // a1 <= a2; equal for the middle block of an odd T
   const int n1 = T - a1, n2 = (a2 != a1) ? T - a2 : 0;
-  const int U = n1 + n2, U0 = (U + 1) / 2;
-  const int lo = half ? U0 : 0, hi = half ? U : U0;
+  const int U = n1 + n2;
+  const int lo = part * U / parts, hi = (part + 1) * U / parts;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WPR, wn = w % WPR;
   const int q = lane >> 4, r = lane & 15;
-  double ra[A_CH][8], rb[B_CH][8];
   doublex4 acc[TM][TN];
   double qs[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) qs[j] = 0.0;
 
-  // acc = H[row block][k blocks kb0..kb1) . X[chain tile][same k]^T
-  auto gemm = [&](int row, int kb0, int kb1) {
-    const double* A = H + (int64_t)row * BM * ldh;
-    const int kt0 = kb0 * KB, kt1 = min(kb1 * KB, KT);
+  // up to two segments per row block: its diagonal block (weight 1, with the
+  // b term) and the blocks beyond it (weight 2)
+  int row = a1, kb = a1 + lo, kend = min(a1 + hi, T), left = hi - lo;
+  if (lo >= n1) {
+    row = a2;
+    kb = a2 + lo - n1;
+    kend = T;
+  }
+#pragma unroll 1
+  while (left > 0) {
+    const bool diag = kb == row;
+    const int k1 = diag ? kb + 1 : min(kend, kb + left);
+    Tile::run(H + (int64_t)row * BM * ldh, ldh, X + n_blk * ldx, ldx, kb * KB, min(k1 * KB, KT), smem, acc);
+    // qs[j] += sum over the lane's rows m of x[n][m] (weight acc - 2 b_m [diagonal block])
+    const double wt = diag ? 1.0 : 2.0;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
-    auto gload = [&](int kt) {
+      for (int v = 0; v < 4; ++v) {
+        const int64_t m = (int64_t)row * BM + wm * WM + i * 16 + q + 4 * v;
+        if (m >= d) continue;
+        const double b2 = diag ? 2.0 * hb[m] : 0.0;
 #pragma unroll
-      for (int i = 0; i < A_CH; ++i) {
-        const int c = tid + i * NT, rr = c >> 1, col = (c & 1) * 8;
-        ld8(A + (int64_t)rr * ldh + (int64_t)kt * BK + col, ra[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + i * NT, rr = c >> 1, col = (c & 1) * 8;
-        ld8(X + (n_blk + rr) * ldx + (int64_t)kt * BK + col, rb[i]);
-      }
-    };
-    gload(kt0);
-    for (int kt = kt0; kt < kt1; ++kt) {
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < A_CH; ++i) {
-        const int c = tid + i * NT, rr = c >> 1, col = (c & 1) * 8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) As[rr * LDS + col + e] = ra[i][e];
-      }
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + i * NT, rr = c >> 1, col = (c & 1) * 8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) Bs[rr * LDS + col + e] = rb[i][e];
-      }
-      __syncthreads();
-      if (kt + 1 < kt1) gload(kt + 1);
-      double af[TM][4], bfr[TN][4];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const double* src = &As[(wm * WM + i * 16 + r) * LDS + 4 * q];
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) af[i][s4] = src[s4];
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const double* src = &Bs[(wn * WN + j * 16 + r) * LDS + 4 * q];
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) bfr[j][s4] = src[s4];
-      }
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][s4], bfr[j][s4], acc[i][j], 0, 0, 0);
-    }
-  };
-  // qs[j] += sum over the lane's rows m of x[n][m] (wt acc - 2 b_m [diagonal block])
-  auto flush = [&](int row, double wt, bool diag) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t m0 = (int64_t)row * BM + wm * WM + i * 16 + q;
-        const int64_t n = n_blk + wn * WN + j * 16 + r;
-        if (n >= N) continue;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int64_t m = m0 + 4 * v;
-          if (m >= d) continue;
-          const double xv = (double)X[n * ldx + m];
-          qs[j] += xv * (wt * acc[i][j][v] - (diag ? 2.0 * hb[m] : 0.0));
+        for (int j = 0; j < TN; ++j) {
+          const int64_t n = n_blk + wn * WN + j * 16 + r;
+          if (n < N) qs[j] += (double)X[n * ldx + m] * (wt * acc[i][j][v] - b2);
         }
       }
-  };
-  for (int sg = 0; sg < 2; ++sg) {
-    const int row = sg ? a2 : a1, base = sg ? n1 : 0, cnt = sg ? n2 : n1;
-    const int s0 = max(lo, base) - base, s1 = min(hi, base + cnt) - base;
-    if (s0 >= s1) continue;
-    int kb0 = row + s0;
-    const int kb1 = row + s1;
-    if (kb0 == row) {
-      gemm(row, kb0, kb0 + 1);
-      flush(row, 1.0, true);
-      ++kb0;
-    }
-    if (kb0 < kb1) {
-      gemm(row, kb0, kb1);
-      flush(row, 2.0, false);
+    left -= k1 - kb;
+    kb = k1;
+    if (kb >= T) {   // the pair's second row block
+      row = a2;
+      kb = a2;
+      kend = T;
     }
   }
+  __syncthreads();
+  double* red = smem;   // [BM / WM][4][BN]
 #pragma unroll
-  for (int j = 0; j < TN; ++j) red[wm][q][wn * WN + j * 16 + r] = qs[j];
+  for (int j = 0; j < TN; ++j) red[(wm * 4 + q) * BN + wn * WN + j * 16 + r] = qs[j];
   __syncthreads();
   for (int col = tid; col < BN; col += NT) {
     double sum = 0.0;
 #pragma unroll
-    for (int a = 0; a < BM / WM; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) sum += red[a][b][col];
-    if (n_blk + col < N) partial[(int64_t)blockIdx.x * ldp + n_blk + col] = sum;
+    for (int a = 0; a < (BM / WM) * 4; ++a) sum += red[a * BN + col];
+    if (n_blk + col < N) partial[(int64_t)item * ldp + n_blk + col] = sum;
   }
-}
-
-static size_t split_elems_f64(int M, int N, int K, int n_cu) {
-  const SplitPlan pl = plan_split(F64_BM, F64_BN, M, N, K, n_cu, true, 16);
-  return pl.split() ? (size_t)pl.SPL * N * pl.TR : 0;
 }
 
 // Workspace for the split tail: float32 partial planes, or null (no split);
@@ -1221,11 +1318,17 @@ static void launch_bf16(Chains& c, int cfg, int split, const uint16_t* A, int64_
 }
 
 size_t gemm_split_workspace_f64(const Problem& p, int64_t B) {
-  if (p.op != 1 || !p.split_tail) return 0;
-  const int n = (int)p.n, d = (int)p.d;
-  size_t e = split_elems_f64(n, (int)B, (int)p.ldg, p.n_cu);        // endpoint, FP64 residual
-  e = std::max(e, split_elems_f64(d, (int)B, (int)round_up(d, 64), p.n_cu));   // premultiplied endpoint
-  if (p.precision == HMC_F64) e = std::max(e, split_elems_f64(d, (int)B, (int)p.ldgt, p.n_cu));
+  if (p.op != 1 || !p.split_tail || p.resolved_engine() != HMC_ENGINE_GEMM) return 0;
+  const int n = (int)p.n, d = (int)p.d, b = (int)B;
+  auto elems = [&](int M, int64_t K) { return f64_ws_elems(plan_f64(M, b, (int)K, p.n_cu, true), b); };
+  size_t e = 0;
+  if (!endpoint_premult(p)) e = std::max(e, elems(n, p.ldg));            // residual endpoint
+  else if (!p.premult_sym) e = std::max(e, elems(d, p.ldg));             // premultiplied endpoint over all of H
+  if (p.precision == HMC_F64) {
+    e = std::max(e, elems(n, p.ldg));                                    // residual
+    e = std::max(e, elems(d, p.ldgt));                                   // gradient
+    if (traj_premult(p)) e = std::max(e, elems(d, p.ldg));               // premultiplied stage
+  }
   return e;
 }
 
@@ -1353,12 +1456,13 @@ static void premult_kick_drift(Chains& c, double kick, double drift, double drif
     launch_bf16(c, p.gemm_cfg_grad, 1, p.Hh, p.ldh, c.dxp[cur], nullptr, c.ldx, d, B, (int)p.ldh, e, 4, 7, true);
     c.dx_cur = 1 - cur;
   } else {
-    // FP64: g = H x - b from a copy of the positions (the epilogue updates xt)
+    // FP64: g = H x - b; the GEMM reads one buffer of positions while the
+    // epilogue writes the other (no copy per stage)
     hipEvent_t ev;
     time_begin(c, 4, ev);
-    HMC_HIP(hipMemcpyAsync(c.xs, c.xt, (size_t)c.B_pad * c.ldx * 8, hipMemcpyDeviceToDevice, p.stream));
+    std::swap(c.xt, c.xs);
     EpiLeap<double> e{(double*)c.xt, (double*)c.pt, nullptr, nullptr, c.ldx, c.eps, c.beta, kick, drift, drift2,
-                      md, d, B, nullptr, nullptr, p.hb};
+                      md, d, B, nullptr, nullptr, p.hb, nullptr, nullptr, (const double*)c.xs};
     launch_f64(c, (const double*)p.H, p.ldh, (const double*)c.xs, c.ldx, d, B, (int)p.ldh, e);
     time_end(c, 4, ev);
   }
@@ -1424,11 +1528,49 @@ bool endpoint_premult(const Problem& p) {
   return p.n > p.d && h_bytes <= 16.0 * 1024 * 1024 * 1024;
 }
 
-int64_t endpoint_blocks(const Chains& c) {
+// How the endpoint runs for this chain set, and the rows of partial sums it
+// writes (at most c.n_mblocks where the buffer is the caller's bound).
+struct EndpointPlan {
+  int64_t rows = 0;
+  int parts = 0;      // k_quad_sym pieces per pair, or 0: plan of the GEMM
+  F64Plan gemm;
+};
+static EndpointPlan endpoint_plan(const Chains& c) {
   const Problem& p = *c.p;
-  if (!endpoint_premult(p)) return (p.n + F64_BM - 1) / F64_BM;
-  const int64_t T = (p.d + F64_BM - 1) / F64_BM;
-  return p.premult_sym ? 2 * ((T + 1) / 2) : T;   // k_quad_sym items, or row blocks of H
+  const int B = (int)c.B;
+  EndpointPlan e;
+  const bool pm = endpoint_premult(p);
+  if (pm && p.premult_sym) {
+    // pieces until every CU has two blocks
+    const int64_t T = (p.d + QS_BM - 1) / QS_BM, pairs = (T + 1) / 2;
+    const int bn = B <= 16 ? 16 : 64;
+    const int64_t tiles = pairs * ((B + bn - 1) / bn);
+    e.parts = 1;
+    while (e.parts < QS_PARTS && tiles * e.parts < 2 * (int64_t)p.n_cu && 2 * e.parts <= T &&
+           2 * e.parts * pairs <= c.n_mblocks)
+      e.parts *= 2;
+    e.rows = pairs * e.parts;
+    return e;
+  }
+  const int M = (int)(pm ? p.d : p.n), K = (int)p.ldg;
+  e.gemm = chains_plan_f64(c, M, B, K);
+  auto rows = [&] {
+    return e.gemm.SPL > 1 ? e.gemm.TR / 128 : (M + f64_bm(e.gemm.cfg) - 1) / (int64_t)f64_bm(e.gemm.cfg);
+  };
+  if (rows() > c.n_mblocks) {
+    e.gemm.cfg = F64_128x128;
+    e.gemm.SPL = 1;
+  }
+  e.rows = rows();
+  return e;
+}
+
+int64_t endpoint_blocks(const Chains& c) { return endpoint_plan(c).rows; }
+
+// rows of endpoint partial sums a chain set allocates
+int64_t endpoint_max_blocks(const Problem& p) {
+  const int64_t T = (p.d + QS_BM - 1) / QS_BM;
+  return std::max({round_up(p.n, 32) / 32, p.d_pad / 32, QS_PARTS * ((T + 1) / 2)});
 }
 
 double endpoint_const(const Problem& p) { return p.misfit_const + (endpoint_premult(p) ? 0.5 * p.dtd : 0.0); }
@@ -1461,7 +1603,7 @@ static void build_premult_t(Chains& c) {
   std::vector<void*> tmp;
   try {
     double* W = (double*)dev_alloc(tmp, (size_t)p.d_pad * p.ldgt * 8);
-    double* v = (double*)dev_alloc(tmp, (size_t)F64_BN * p.ldgt * 8);
+    double* v = (double*)dev_alloc(tmp, (size_t)F64_MAX_BN * p.ldgt * 8);
     const dim3 grid((unsigned)std::min<int64_t>((p.ldgt + 255) / 256, 64), (unsigned)std::min<int64_t>(p.d_pad, 65535));
     hipLaunchKernelGGL(k_scale_cols<TG>, grid, dim3(256), 0, p.stream, Gt, p.ldgt, p.d_pad, p.n, p.var, W);
     HMC_HIP(hipGetLastError());
@@ -1498,28 +1640,40 @@ static void build_premult(Chains& c) {
 void gemm_endpoint(Chains& c, const void* X, int x_dtype) {
   Problem& p = *c.p;
   const int n = (int)p.n, B = (int)c.B;
-  HMC_REQUIRE(endpoint_blocks(c) <= c.n_mblocks, HMC_ERR_STATE, "endpoint partial buffer too small");
+  const EndpointPlan ep = endpoint_plan(c);
+  HMC_REQUIRE(ep.rows <= c.n_mblocks, HMC_ERR_STATE, "endpoint partial buffer too small");
   if (endpoint_premult(p)) {
     if (!p.H) build_premult(c);
     const int d = (int)p.d;
     hipEvent_t ev;
     time_begin(c, 1, ev);
     if (p.premult_sym) {
-      constexpr int NT = (F64_BM / F64_WM) * (F64_BN / F64_WN) * 64;
-      const int64_t T = (p.d + F64_BM - 1) / F64_BM;
-      const dim3 grid((unsigned)(2 * ((T + 1) / 2)), (unsigned)((B + F64_BN - 1) / F64_BN));
-      if (x_dtype == HMC_F32)
-        hipLaunchKernelGGL(k_quad_sym<float>, grid, dim3(NT), 0, p.stream, (const double*)p.H, p.ldh,
-                           (const float*)X, c.ldx, p.hb, d, B, c.partial, c.B_pad);
-      else
-        hipLaunchKernelGGL(k_quad_sym<double>, grid, dim3(NT), 0, p.stream, (const double*)p.H, p.ldh,
-                           (const double*)X, c.ldx, p.hb, d, B, c.partial, c.B_pad);
+      const int64_t pairs = ((p.d + QS_BM - 1) / QS_BM + 1) / 2;
+      auto go = [&](auto bn, auto wm, auto wn, auto bk, auto* x) {
+        constexpr int BN = decltype(bn)::value, WM = decltype(wm)::value, WN = decltype(wn)::value;
+        using TX = std::remove_const_t<std::remove_pointer_t<decltype(x)>>;
+        const dim3 grid((unsigned)grid_for((int)(pairs * ep.parts), (B + BN - 1) / BN));
+        hipLaunchKernelGGL((k_quad_sym<BN, WM, WN, decltype(bk)::value, TX>), grid,
+                           dim3((QS_BM / WM) * (BN / WN) * 64), 0, p.stream, (const double*)p.H, p.ldh, x, c.ldx, p.hb,
+                           d, B, ep.parts, c.partial, c.B_pad);
+      };
+      using std::integral_constant;
+      auto by_b = [&](auto* x) {
+        if (B <= 16)
+          go(integral_constant<int, 16>{}, integral_constant<int, 16>{}, integral_constant<int, 16>{},
+             integral_constant<int, 32>{}, x);
+        else
+          go(integral_constant<int, 64>{}, integral_constant<int, 32>{}, integral_constant<int, 32>{},
+             integral_constant<int, 16>{}, x);
+      };
+      if (x_dtype == HMC_F32) by_b((const float*)X);
+      else by_b((const double*)X);
       HMC_HIP(hipGetLastError());
     } else if (x_dtype == HMC_F32) {
-      launch_f64(c, (const double*)p.H, p.ldh, (const float*)X, c.ldx, d, B, (int)p.ldh,
+      launch_f64(c, ep.gemm, (const double*)p.H, p.ldh, (const float*)X, c.ldx, d, B, (int)p.ldh,
                  EpiQuad<float>{(const float*)X, c.ldx, p.hb, c.partial, c.B_pad, d, B});
     } else {
-      launch_f64(c, (const double*)p.H, p.ldh, (const double*)X, c.ldx, d, B, (int)p.ldh,
+      launch_f64(c, ep.gemm, (const double*)p.H, p.ldh, (const double*)X, c.ldx, d, B, (int)p.ldh,
                  EpiQuad<double>{(const double*)X, c.ldx, p.hb, c.partial, c.B_pad, d, B});
     }
     time_end(c, 1, ev);
@@ -1530,19 +1684,19 @@ void gemm_endpoint(Chains& c, const void* X, int x_dtype) {
   time_begin(c, 1, ev);
   if (p.tgt_dtype == HMC_BF16) {
     if (x_dtype == HMC_F32)
-      launch_f64(c, (const uint16_t*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const uint16_t*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
     else
-      launch_f64(c, (const uint16_t*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const uint16_t*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
   } else if (p.tgt_dtype == HMC_F32) {
     if (x_dtype == HMC_F32)
-      launch_f64(c, (const float*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const float*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
     else
-      launch_f64(c, (const float*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const float*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
   } else {
     if (x_dtype == HMC_F32)
-      launch_f64(c, (const double*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const double*)p.G_tgt, p.ldg, (const float*)X, c.ldx, n, B, (int)p.ldg, e);
     else
-      launch_f64(c, (const double*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
+      launch_f64(c, ep.gemm, (const double*)p.G_tgt, p.ldg, (const double*)X, c.ldx, n, B, (int)p.ldg, e);
   }
   time_end(c, 1, ev);
 }

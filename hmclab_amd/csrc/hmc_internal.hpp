@@ -137,8 +137,9 @@ struct Chains {
   float* yref = nullptr;
   bool anchor_ready = false;
   // premultiplied bf16: the planes of x - x_ref alternate between two buffers
-  // (a stage's GEMM reads one while its epilogue writes the other); FP64 reads
-  // a copy xs of the positions while the epilogue updates xt
+  // (a stage's GEMM reads one while its epilogue writes the other); FP64
+  // positions alternate between xt and xs in the same way (the two pointers are
+  // exchanged per stage: xt always holds the latest positions)
   uint16_t* dxp[2] = {nullptr, nullptr};
   int dx_cur = 0;
   void* xs = nullptr;
@@ -254,6 +255,7 @@ size_t gemm_split_workspace(const Problem& p, int64_t B);      // float elements
 size_t gemm_split_workspace_f64(const Problem& p, int64_t B);  // double elements
 bool endpoint_premult(const Problem& p);      // endpoint misfit uses H (dense GEMM engine)
 int64_t endpoint_blocks(const Chains& c);     // rows of the endpoint partial sums
+int64_t endpoint_max_blocks(const Problem& p);// rows to allocate for them
 double endpoint_const(const Problem& p);      // constant added to every misfit
 // Trajectory gradient + fused kick/drift for every chain:
 //   p -= kick*eps*g(xt); xt += drift*eps*Minv p; corrector; [xt += drift2*eps*Minv p; corrector]
