@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <numeric>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "hmc_internal.hpp"
@@ -18,14 +19,14 @@ struct hmc_surrogate;
 namespace hmc {
 
 // ---------------------------------------------------------------------------
-// generic GEMM: C[m][n] = alpha * sum_k A(m,k) B(n,k) + beta * C[m][n]
+// FP32 GEMM (mode f32): C[m][n] = alpha * sum_k A(m,k) B(n,k) + beta * C[m][n]
 //   A(m,k) = TA ? A[k*lda + m] : A[m*lda + k];  B(n,k) = TB ? B[k*ldb + n] : B[n*ldb + k]
 // 64x64x32 tiles, 256 threads; dimensions must be multiples of the tile (the
 // surrogate pads every dimension to 64).
 // ---------------------------------------------------------------------------
 constexpr int SG_T = 64, SG_K = 32;
 
-template <bool TA, bool TB, bool MFMA>
+template <bool TA, bool TB>
 __global__ __launch_bounds__(256) void k_sgemm(const float* __restrict__ A, int64_t lda,
                                                const float* __restrict__ B, int64_t ldb,
                                                float* __restrict__ C, int64_t ldc, int K,
@@ -49,60 +50,28 @@ __global__ __launch_bounds__(256) void k_sgemm(const float* __restrict__ A, int6
       for (int e = 0; e < 8; ++e) S[r + e][kk] = src[e];
     }
   };
-  if constexpr (MFMA) {
-    // 4 waves in 2 x 2, each one 32x32 bf16 MFMA tile
-    const int lane = tid & 63, w = tid >> 6, wm = w >> 1, wn = w & 1;
-    const int q = lane >> 5, r = lane & 31;
-    floatx16 acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    for (int k0 = 0; k0 < K; k0 += SG_K) {
-      __syncthreads();
-      stage(A, lda, TA, m0, k0, As);
-      stage(B, ldb, TB, n0, k0, Bs);
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        bf16x8 a, b;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          a[e] = (__bf16)As[wm * 32 + r][16 * s + 8 * q + e];
-          b[e] = (__bf16)Bs[wn * 32 + r][16 * s + 8 * q + e];
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t m = m0 + wm * 32 + 8 * (v >> 2) + 4 * q + (v & 3);
-      const int64_t n = n0 + wn * 32 + r;
-      float* cp = C + m * ldc + n;
-      *cp = alpha * acc[v] + (beta != 0.f ? beta * *cp : 0.f);
-    }
-  } else {
-    // SIMT: each thread a 4 x 4 micro tile
-    const int tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += SG_K) {
-      __syncthreads();
-      stage(A, lda, TA, m0, k0, As);
-      stage(B, ldb, TB, n0, k0, Bs);
-      __syncthreads();
+  // each thread a 4 x 4 micro tile
+  const int tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < K; k0 += SG_K) {
+    __syncthreads();
+    stage(A, lda, TA, m0, k0, As);
+    stage(B, ldb, TB, n0, k0, Bs);
+    __syncthreads();
 #pragma unroll 8
-      for (int k = 0; k < SG_K; ++k)
+    for (int k = 0; k < SG_K; ++k)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] += As[tm + i][k] * Bs[tn + j][k];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float* cp = C + (m0 + tm + i) * ldc + n0 + tn + j;
-        *cp = alpha * acc[i][j] + (beta != 0.f ? beta * *cp : 0.f);
-      }
+        for (int j = 0; j < 4; ++j) acc[i][j] += As[tm + i][k] * Bs[tn + j][k];
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float* cp = C + (m0 + tm + i) * ldc + n0 + tn + j;
+      *cp = alpha * acc[i][j] + (beta != 0.f ? beta * *cp : 0.f);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -265,19 +234,29 @@ __global__ void k_sum(const float* v, int64_t n, float* out) {
   if (threadIdx.x == 0) out[0] = red[0];
 }
 
-__global__ void k_adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, float b1,
-                       float b2, float c1, float c2, float eps) {
+// Adam step of parameter i with gradient gi; returns the new value
+struct AdamStep {
+  float *w, *m, *v;
+  float lr, b1, b2, c1, c2, eps;
+  // moments and value wo, mo, vo as loaded by the caller
+  __device__ __forceinline__ float apply(int64_t i, float gi, float wo, float mo, float vo) const {
+    const float mi = b1 * mo + (1.f - b1) * gi;
+    const float vi = b2 * vo + (1.f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float wi = wo - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    return wi;
+  }
+  __device__ __forceinline__ float apply(int64_t i, float gi) const { return apply(i, gi, w[i], m[i], v[i]); }
+};
+
+__global__ void k_adam(AdamStep a, const float* g, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  if (i < n) a.apply(i, g[i]);
 }
 
-// gather + normalise training rows: Xn[b] = (X[idx[b]] - xm)/xs ; Tn[b] = T[idx[b]] * xs / fs
+// gather normalised training rows: Xn[b] = X[idx[b]], Tn[b] = T[idx[b]], yb[b] = y[idx[b]]
 __global__ void k_gather(const float* Xall, const float* Tall, const float* yall, const int32_t* idx,
                          float* Xn, float* Tn, float* yb, int64_t Dp, int64_t rows) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -290,9 +269,606 @@ __global__ void k_gather(const float* Xall, const float* Tall, const float* yall
 }
 
 // ---------------------------------------------------------------------------
+// bf16 products of the evaluation and training passes
+//   C[m][n] = sum_k A[m][k] B[n][k]   (+ a second product, added after it)
+// on bf16 planes whose rows are k-contiguous, FP32 accumulation in ascending k
+// (v_mfma_f32_32x32x16_bf16, one 16-deep step after the other, so a result does
+// not depend on the tile).  A block of WM x WN waves computes 32 WM x 32 WN
+// outputs; its operand tiles stream global -> LDS with direct-to-LDS loads
+// through an S-stage ring of 64-wide k-tiles, rows swizzled in 16-byte chunks
+// by (row & 7).
+//
+// What bounds it: these products are small (256 x 512 outputs are 128 tiles of
+// 32 x 32), so each block's chain of k-tiles and its loads in flight, not the
+// matrix cores.  One wave per 32 x 32 tile keeps 7 k-tiles (56 KB) in flight
+// and needs no barrier; in a long product a second wave issues all the loads, so
+// the first runs only LDS reads and MFMAs; 64 x 64 blocks take the products with
+// many outputs.  The fragments of a k-tile are read while the MFMAs of the one
+// before run, and the two products of a weight gradient are two loops (a test
+// per k-tile made the accumulators travel through plain registers).
+// 256 x 512 x 8192: 30 us (194 us with 64 x 64 tiles staged through registers as
+// float32); 256 x 512 x 512: 7 us (15 us).
+// ---------------------------------------------------------------------------
+#define HMC_LDS __attribute__((address_space(3)))
+
+template <int N>
+__device__ inline void sur_wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt out of range");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
+}
+
+struct SurOperands {
+  const uint16_t *a = nullptr, *b = nullptr;
+  int64_t lda = 0, ldb = 0;
+  int K = 0;
+};
+
+template <int WM, int WN, int LW, int S, class Epi>
+__global__ __launch_bounds__((WM * WN + LW) * 64) void k_sur_gemm(SurOperands p0, SurOperands p1, int gm, int gn,
+                                                                  Epi epi) {
+  constexpr int BK = 64, CW = WM * WN, NW = CW + LW, BM = 32 * WM, BN = 32 * WN;
+  constexpr int NL = LW > 0 ? LW : CW;   // waves that load
+  constexpr int A_GROUPS = BM / 8, GROUPS = (BM + BN) / 8, GPW = GROUPS / NL;   // 1 KB loads
+  constexpr int STAGE = (BM + BN) * BK;
+  static_assert(GROUPS % NL == 0 && GPW * (S - 2) < 64, "load groups");
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[S * STAGE];
+
+  // tiles dealt to the XCDs in contiguous n-major ranges (an XCD reads its own
+  // rows of B and all of the smaller A)
+  const int T = gm * gn, chunk = (T + 7) / 8, t = ((int)blockIdx.x % 8) * chunk + (int)blockIdx.x / 8;
+  if (t >= T) return;
+  const int64_t m_blk = (int64_t)(t % gm) * BM, n_blk = (int64_t)(t / gm) * BN;
+  const int tid = threadIdx.x, lane = tid & 63, w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool loader = LW == 0 || w >= CW, computes = LW == 0 || w < CW;
+  const int lw = LW > 0 ? w - CW : w;    // index among the loading waves
+  const int wm = w / WN, wn = w % WN;
+  const int q = lane >> 5, r = lane & 31, lrow = lane >> 3;
+
+  // this lane's source of each of the wave's load groups, advanced per k-tile
+  const int nk0 = p0.K / BK, nk = nk0 + p1.K / BK;
+  const uint16_t* src[GPW];
+  auto aim = [&](const SurOperands& p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < GPW; ++i) {
+      const int g = lw * GPW + i;
+      const bool is_a = g < A_GROUPS;
+      const int row = (is_a ? g : g - A_GROUPS) * 8 + lrow;
+      const uint16_t* base = is_a ? p.a : p.b;
+      const int64_t at = is_a ? (m_blk + row) * p.lda : (n_blk + row) * p.ldb;
+      src[i] = base + at + ((lane & 7) ^ (row & 7)) * 8;
+    }
+  };
+  auto issue = [&](int kt, int st) __attribute__((always_inline)) {
+    if (kt == nk0) aim(p1);
+    uint16_t* stage = smem + st * STAGE;
+#pragma unroll
+    for (int i = 0; i < GPW; ++i) {
+      __builtin_amdgcn_global_load_lds((const void*)src[i], (HMC_LDS void*)(stage + (lw * GPW + i) * 8 * BK), 16, 0, 0);
+      src[i] += BK;
+    }
+  };
+  if (loader) {
+    aim(p0);
+#pragma unroll
+    for (int s0 = 0; s0 < S - 1; ++s0)
+      if (s0 < nk) issue(s0, s0);
+  }
+  floatx16 acc, first;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = first[v] = 0.f;
+  bf16x8 af[2][4] = {}, bf[2][4] = {};
+  const int ra = wm * 32 + r, rb = wn * 32 + r;
+  auto mfmas = [&](auto set) __attribute__((always_inline)) {
+    constexpr int p = decltype(set)::value;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[p][s], bf[p][s], acc, 0, 0, 0);
+  };
+  // k-tile kt with its fragments in set p; the MFMAs of the k-tile before it
+  // (set 1 - p, unless kt is the product's first) run while they are read
+  auto tile = [&](int kt, auto set, auto is_first) __attribute__((always_inline)) {
+    constexpr int p = decltype(set)::value;
+    if (loader) {
+      if (kt + S - 2 < nk) sur_wait_vmcnt<GPW * (S - 2)>();
+      else sur_wait_vmcnt<0>();
+    }
+    // this wave's LDS reads of the stage about to be refilled have returned
+    // (naming the fragments keeps the compiler from moving their reads past
+    // this point); with several waves, all of them have passed the barrier
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(af[1 - p][0]), "+v"(af[1 - p][1]), "+v"(af[1 - p][2]), "+v"(af[1 - p][3]), "+v"(bf[1 - p][0]),
+                   "+v"(bf[1 - p][1]), "+v"(bf[1 - p][2]), "+v"(bf[1 - p][3])
+                 :
+                 : "memory");
+    if constexpr (NW > 1) {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    if (computes) {
+      const uint16_t* As = smem + (kt % S) * STAGE;
+      const uint16_t* Bs = As + BM * BK;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int c = 2 * s + q;   // k = 16 s + 8 q + e
+        af[p][s] = *reinterpret_cast<const bf16x8*>(&As[ra * BK + ((c ^ (ra & 7)) << 3)]);
+        bf[p][s] = *reinterpret_cast<const bf16x8*>(&Bs[rb * BK + ((c ^ (rb & 7)) << 3)]);
+      }
+      if constexpr (!decltype(is_first)::value) mfmas(std::integral_constant<int, 1 - p>{});
+    }
+    if (loader && kt + S - 1 < nk) issue(kt + S - 1, (kt + S - 1) % S);
+  };
+  using Set0 = std::integral_constant<int, 0>;
+  using Set1 = std::integral_constant<int, 1>;
+  auto product = [&](int kt, int end) __attribute__((always_inline)) {
+    tile(kt, Set0{}, std::true_type{});
+    for (++kt; kt + 2 <= end; kt += 2) {
+      tile(kt, Set1{}, std::false_type{});
+      tile(kt + 1, Set0{}, std::false_type{});
+    }
+    if (kt < end) {
+      tile(kt, Set1{}, std::false_type{});
+      if (computes) mfmas(Set1{});
+    } else if (computes) {
+      mfmas(Set0{});
+    }
+  };
+  product(0, nk0);
+  if (nk > nk0) {
+    first = acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    product(nk0, nk);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = acc[v] + first[v];
+  }
+  if (!computes) return;
+  // lane (q, r) holds rows 8 g + 4 q + v (g, v = 0..3) of column r
+  epi.apply(m_blk + wm * 32, 4 * q, n_blk + wn * 32 + r, acc);
+}
+
+// the lane's 16 values of src at rows b0 + 8 g + q4 + v of column h, loaded
+// before an epilogue's first store (a store between them would order them)
+__device__ __forceinline__ floatx16 load16(const float* src, int64_t b0, int q4, int64_t h, int64_t ld) {
+  floatx16 o;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o[i] = src[(b0 + 8 * (i / 4) + q4 + i % 4) * ld + h];
+  return o;
+}
+
+// 4 consecutive batch rows of one column as bf16: the transposed plane's 8-byte
+// store
+__device__ __forceinline__ void put_t4(uint16_t* pT, int64_t o, const float v[4]) {
+  const uint32_t h0 = f32_to_bf16_bits(v[0]), h1 = f32_to_bf16_bits(v[1]), h2 = f32_to_bf16_bits(v[2]),
+                 h3 = f32_to_bf16_bits(v[3]);
+  *reinterpret_cast<uint2*>(&pT[o]) = uint2{h0 | (h1 << 16), h2 | (h3 << 16)};
+}
+
+// Epilogues: m = batch row b, n = column; rows b0 + 8 g + q4 + v.
+
+// Z1 = acc + b1; A1 = silu(Z1), S1 = silu'(Z1)
+struct SurZ1 {
+  const float* bias;
+  float *z, *s;
+  uint16_t *a, *aT;   // aT may be null (evaluation)
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const float bh = bias[h];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float av[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        const float zz = acc[4 * g + v] + bh;
+        z[o] = zz;
+        s[o] = dsilu_f(zz);
+        av[v] = silu_f(zz);
+        a[o] = f32_to_bf16_bits(av[v]);
+      }
+      if (aT) put_t4(aT, h * R + b0 + 8 * g + q4, av);
+    }
+  }
+};
+
+// Z2 = acc + b2; A2 = silu(Z2), S2 = silu'(Z2), U2 = S2 w3
+struct SurZ2 {
+  const float *bias, *w3;
+  float *z, *a, *s;
+  uint16_t *u, *uT;
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const float bh = bias[h], wh = w3[h];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float uv[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        const float zz = acc[4 * g + v] + bh;
+        z[o] = zz;
+        a[o] = silu_f(zz);
+        const float ss = dsilu_f(zz);
+        s[o] = ss;
+        uv[v] = ss * wh;
+        u[o] = f32_to_bf16_bits(uv[v]);
+      }
+      if (uT) put_t4(uT, h * R + b0 + 8 * g + q4, uv);
+    }
+  }
+};
+
+// V1 = acc; U1 = S1 V1
+struct SurV1 {
+  const float* s1;
+  float* v1;
+  uint16_t *u, *uT;
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const floatx16 ss = load16(s1, b0, q4, h, H);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float uv[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        v1[o] = acc[4 * g + v];
+        uv[v] = ss[4 * g + v] * acc[4 * g + v];
+        u[o] = f32_to_bf16_bits(uv[v]);
+      }
+      if (uT) put_t4(uT, h * R + b0 + 8 * g + q4, uv);
+    }
+  }
+};
+
+// input gradient of the evaluation: out[b][j] = acc gscale_j (raw units, FP64)
+struct SurEvalGrad {
+  const float* gscale;
+  double* out;
+  int64_t D, B;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t j, const floatx16& acc) const {
+    if (j >= D) return;
+    const double gs = (double)gscale[j];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t b = b0 + 8 * g + q4 + v;
+        if (b < B) out[b * D + j] = (double)acc[4 * g + v] * gs;
+      }
+  }
+};
+
+// training: E = acc - t, dG = 2 beta / D E / R, tile sums of E^2 per batch row
+struct SurResid {
+  const float* t;        // [.][Dp], row idx[b]
+  const int32_t* idx;    // or null: row b
+  uint16_t *dg, *dgT;
+  float* lpart;          // [Dp / 32][R]
+  int64_t D, Dp, R;
+  float beta;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t j, const floatx16& acc) const {
+    const int r = threadIdx.x & 31;
+    float tt[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int64_t b = b0 + 8 * (i / 4) + q4 + i % 4;
+      tt[i] = t[(idx ? idx[b] : b) * Dp + j];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float dv[4], e2[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t b = b0 + 8 * g + q4 + v;
+        const float e = (j < D) ? acc[4 * g + v] - tt[4 * g + v] : 0.f;
+        dv[v] = 2.f * beta / (float)D * e / (float)R;
+        e2[v] = e * e;
+        dg[b * Dp + j] = f32_to_bf16_bits(dv[v]);
+      }
+      put_t4(dgT, j * R + b0 + 8 * g + q4, dv);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) e2[v] += __shfl_xor(e2[v], off, 32);
+        if (r == 0) lpart[(j / 32) * R + b0 + 8 * g + q4 + v] = e2[v];
+      }
+    }
+  }
+};
+
+// dU1 = acc; dS1 = dU1 V1, dV1 = dU1 S1
+struct SurDU1 {
+  const float *v1, *s1;
+  float* ds1;
+  uint16_t *dv, *dvT;
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const floatx16 vv = load16(v1, b0, q4, h, H), ss = load16(s1, b0, q4, h, H);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float dd[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        ds1[o] = acc[4 * g + v] * vv[4 * g + v];
+        dd[v] = acc[4 * g + v] * ss[4 * g + v];
+        dv[o] = f32_to_bf16_bits(dd[v]);
+      }
+      put_t4(dvT, h * R + b0 + 8 * g + q4, dd);
+    }
+  }
+};
+
+// dU2 = acc; dZ2 = dU2 w3 silu''(Z2) + df w3 S2
+struct SurDU2 {
+  const float *w3, *z2, *s2, *df;
+  float *du, *dzf;
+  uint16_t *dz, *dzT;
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const floatx16 zz = load16(z2, b0, q4, h, H), ss = load16(s2, b0, q4, h, H), dfb = load16(df, b0, q4, 0, 1);
+    const float wh = w3[h];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float dd[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 4 * g + v;
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        du[o] = acc[i];
+        dd[v] = acc[i] * wh * d2silu_f(zz[i]) + dfb[i] * wh * ss[i];
+        dzf[o] = dd[v];
+        dz[o] = f32_to_bf16_bits(dd[v]);
+      }
+      put_t4(dzT, h * R + b0 + 8 * g + q4, dd);
+    }
+  }
+};
+
+// dA1 = acc; dZ1 = dS1 silu''(Z1) + dA1 S1
+struct SurDA1 {
+  const float *ds1, *z1, *s1;
+  float* dzf;
+  uint16_t* dzT;
+  int64_t H, R;
+  __device__ __forceinline__ void apply(int64_t b0, int q4, int64_t h, const floatx16& acc) const {
+    const floatx16 dd1 = load16(ds1, b0, q4, h, H), zz = load16(z1, b0, q4, h, H), ss = load16(s1, b0, q4, h, H);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float dd[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 4 * g + v;
+        const int64_t o = (b0 + 8 * g + q4 + v) * H + h;
+        dd[v] = fmaf(acc[i], ss[i], dd1[i] * d2silu_f(zz[i]));
+        dzf[o] = dd[v];
+      }
+      put_t4(dzT, h * R + b0 + 8 * g + q4, dd);
+    }
+  }
+};
+
+// weight gradient W[m][n] (m = hidden unit, n = input): stored, or (training)
+// the Adam step and the new weight's planes [m][n] and [n][m]
+struct SurWeight {
+  float* g;            // gradient, or null: Adam
+  AdamStep adam;
+  int64_t off;         // of the matrix in the packed parameters
+  uint16_t *h, *t;     // planes
+  int64_t ld, ldt;     // row strides of W (and plane h) and of plane t
+  __device__ __forceinline__ void apply(int64_t m0, int q4, int64_t n, const floatx16& acc) const {
+    if (g) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) g[off + (m0 + 8 * (i / 4) + q4 + i % 4) * ld + n] = acc[i];
+      return;
+    }
+    const floatx16 wo = load16(adam.w + off, m0, q4, n, ld), mo = load16(adam.m + off, m0, q4, n, ld),
+                   vo = load16(adam.v + off, m0, q4, n, ld);
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      float wv[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 4 * gq + v;
+        const int64_t o = (m0 + 8 * gq + q4 + v) * ld + n;
+        wv[v] = adam.apply(off + o, acc[i], wo[i], mo[i], vo[i]);
+        h[o] = f32_to_bf16_bits(wv[v]);
+      }
+      put_t4(t, n * ldt + m0 + 8 * gq + q4, wv);
+    }
+  }
+};
+
+// f[b] = A2[b] . w3 + b3 (fixed tree); df = 2 alpha (f - y) / R when training
+__global__ void k_sur_head(const float* a2, const float* w3, const float* b3, const float* y, const int32_t* idx,
+                           float alpha, float* f, float* df, int H, int R) {
+  __shared__ float red[256];
+  const int64_t b = blockIdx.x;
+  float acc = 0.f;
+  for (int i = threadIdx.x; i < H; i += 256) acc += a2[b * H + i] * w3[i];
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const float fv = red[0] + b3[0];
+    f[b] = fv;
+    if (df) df[b] = 2.f * alpha * (fv - y[idx ? idx[b] : b]) / (float)R;
+  }
+}
+
+// e2[b] = sum over the column tiles of lpart[tile][b]: 32 batch rows per block,
+// 8 threads each
+__global__ __launch_bounds__(256) void k_sur_e2(const float* __restrict__ lpart, int tiles, int R,
+                                                float* __restrict__ e2) {
+  __shared__ float red[8][32];
+  const int b = threadIdx.x & 31, k = threadIdx.x >> 5;
+  float s = 0.f;
+#pragma unroll 8
+  for (int t = k; t < tiles; t += 8) s += lpart[(int64_t)t * R + blockIdx.x * 32 + b];
+  red[k][b] = s;
+  __syncthreads();
+  if (k == 0) {
+    for (int i = 1; i < 8; ++i) s += red[i][b];
+    e2[blockIdx.x * 32 + b] = s;
+  }
+}
+
+// Column sums over the batch in row order, 32 rows of loads ahead of their
+// sums: block (x, 0) dw3 = sum_b dU2 S2 + df A2, (x, 1) db2 = sum_b dZ2, (x, 2)
+// db1 = sum_b dZ1; block (0, 3) db3 = sum_b df and the batch loss
+// sum_b alpha r^2 + beta / D sum E^2 (e2: k_sur_e2's sums).  Gradients are stored (g) or take their
+// Adam step (g null).  One column per thread and 64 columns per block: the sums
+// are serial chains, so the loads in flight bound them (256 rows of 512
+// columns: 31 us per sum with 256-column blocks and a load per step).
+struct SurFinish {
+  const float *du2, *s2, *a2, *dz2, *dz1, *e2, *f, *y, *df;
+  const int32_t* idx;
+  float* g;
+  AdamStep adam;
+  int64_t ow3, ob2, ob1, ob3;
+  float* loss;
+  int H, R, D;
+  float alpha, beta;
+};
+__global__ __launch_bounds__(64) void k_sur_finish(SurFinish p) {
+  constexpr int U = 32;
+  auto put = [&](int64_t o, float v) {
+    if (p.g) p.g[o] = v;
+    else p.adam.apply(o, v);
+  };
+  const int h = blockIdx.x * 64 + threadIdx.x, which = blockIdx.y;
+  if (which < 3) {   // H and R are multiples of 64
+    float acc = 0.f;
+    if (which == 0) {
+      for (int b0 = 0; b0 < p.R; b0 += U) {
+        float du[U], ss[U], aa[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t o = (int64_t)(b0 + u) * p.H + h;
+          du[u] = p.du2[o];
+          ss[u] = p.s2[o];
+          aa[u] = p.a2[o];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          acc += du[u] * ss[u];
+          acc += p.df[b0 + u] * aa[u];
+        }
+      }
+      put(p.ow3 + h, acc);
+    } else {
+      const float* z = which == 1 ? p.dz2 : p.dz1;
+      for (int b0 = 0; b0 < p.R; b0 += U) {
+        float zz[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) zz[u] = z[(int64_t)(b0 + u) * p.H + h];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += zz[u];
+      }
+      put((which == 1 ? p.ob2 : p.ob1) + h, acc);
+    }
+    return;
+  }
+  if (blockIdx.x != 0) return;
+  // 256 strided sums, then a fixed tree
+  __shared__ float red[2][256];
+  for (int i = threadIdx.x; i < 256; i += 64) {
+    float sd = 0.f, sl = 0.f;
+    for (int b = i; b < p.R; b += 256) {
+      const float r = p.f[b] - p.y[p.idx ? p.idx[b] : b];
+      sd += p.df[b];
+      sl += p.alpha * r * r + p.beta / (float)p.D * p.e2[b];
+    }
+    red[0][i] = sd;
+    red[1][i] = sl;
+  }
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    for (int i = threadIdx.x; i < s; i += 64) {
+      red[0][i] += red[0][i + s];
+      red[1][i] += red[1][i + s];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    put(p.ob3, red[0][0]);
+    *p.loss = red[1][0];
+  }
+}
+
+// bf16 planes of rows idx[b] (or b) of X [.][Dp]: x[b][j] and, transposed
+// through LDS, xT[j][b].  One 64 x 64 tile per block.
+__global__ __launch_bounds__(256) void k_sur_rows(const float* __restrict__ X, const int32_t* __restrict__ idx,
+                                                  int64_t Dp, int64_t R, uint16_t* __restrict__ x,
+                                                  uint16_t* __restrict__ xT) {
+  __shared__ uint16_t tile[64][66];
+  const int64_t j0 = (int64_t)blockIdx.x * 64, b0 = (int64_t)blockIdx.y * 64;
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+  float f[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int64_t b = b0 + r0 + 4 * k;
+    f[k] = X[(idx ? idx[b] : b) * Dp + j0 + c];
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int r = r0 + 4 * k;
+    const uint16_t v = f32_to_bf16_bits(f[k]);
+    x[(b0 + r) * Dp + j0 + c] = v;
+    tile[c][r] = v;
+  }
+  if (!xT) return;
+  __syncthreads();
+  for (int r = r0; r < 64; r += 4) xT[(j0 + r) * R + b0 + c] = tile[r][c];
+}
+
+// parameters without W1's padding columns: W1 [H][D], then the rest
+__global__ void k_sur_pack(const float* __restrict__ p, int64_t H, int64_t D, int64_t Dp, int64_t n,
+                           float* __restrict__ out) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    out[i] = i < H * D ? p[(i / D) * Dp + i % D] : p[i - H * D + H * Dp];
+}
+
+// host rows (f64 [n][D]) -> float32 [n][Dp], zero in the padding columns:
+// mode 0 as given, 1 ((float)v - mean) / scale in float32, 2 (v - mean) / scale
+// in FP64, 3 v scale / fs in FP64
+__global__ void k_sur_load(const double* __restrict__ src, int64_t n, int64_t D, int64_t Dp,
+                           const float* __restrict__ xm, const float* __restrict__ xs, double fs, int mode,
+                           float* __restrict__ dst) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n * Dp; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t b = i / Dp, j = i % Dp;
+    float o = 0.f;
+    if (j < D) {
+      const double v = src[b * D + j];
+      if (mode == 0) o = (float)v;
+      else if (mode == 1) o = ((float)v - xm[j]) / xs[j];
+      else if (mode == 2) o = (float)((v - (double)xm[j]) / (double)xs[j]);
+      else o = (float)(v * (double)xs[j] / fs);
+    }
+    dst[i] = o;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // host object
 // ---------------------------------------------------------------------------
+// Buffers of the bf16 evaluation and training passes, for up to `rows` rows
+struct TrainBufs {
+  int64_t rows = 0;
+  // operand planes: [b][k] and transposed [k][b] (suffix T)
+  uint16_t *x = nullptr, *xT = nullptr, *dg = nullptr, *dgT = nullptr, *a1 = nullptr, *a1T = nullptr, *u2 = nullptr,
+           *u2T = nullptr, *u1 = nullptr, *u1T = nullptr, *dv1 = nullptr, *dv1T = nullptr, *dz2 = nullptr,
+           *dz2T = nullptr, *dz1T = nullptr;
+  float *z1 = nullptr, *s1 = nullptr, *z2 = nullptr, *a2 = nullptr, *s2 = nullptr, *v1 = nullptr, *ds1 = nullptr,
+        *du2 = nullptr, *dz2f = nullptr, *dz1f = nullptr;
+  float *f = nullptr, *df = nullptr, *e2 = nullptr;
+  float* lpart = nullptr;   // [Dp / 32][rows] sums of (grad f - t)^2
+};
+
 struct Surrogate {
+  TrainBufs tb;
   int64_t D = 0, Dp = 0, H = 0;
   int mode = 0;                  // 0 bf16 MFMA, 1 fp32 SIMT
   hipStream_t stream = nullptr;
@@ -337,6 +913,7 @@ struct Surrogate {
   float* b3() { return P + ob3; }
 };
 
+// float32 mode: full-precision copies of every intermediate
 static void ensure_rows(Surrogate& s, int64_t rows) {
   rows = round_up(rows, 64);
   if (rows <= s.Bmax) return;
@@ -351,17 +928,31 @@ static void ensure_rows(Surrogate& s, int64_t rows) {
   s.Bmax = rows;
 }
 
+// bf16 mode: operand planes ([row][k] and, where a product over the batch
+// reads it, the transpose) and the float32 values the epilogues need again
+static void ensure_train_rows(Surrogate& s, int64_t rows) {
+  rows = round_up(rows, 64);
+  TrainBufs& t = s.tb;
+  if (rows <= t.rows) return;
+  auto F = [&](size_t n) { return (float*)dev_alloc(s.owned, n * sizeof(float)); };
+  auto U = [&](size_t n) { return (uint16_t*)dev_alloc(s.owned, n * 2); };
+  const int64_t RD = rows * s.Dp, RH = rows * s.H;
+  t.x = U(RD); t.xT = U(RD); t.dg = U(RD); t.dgT = U(RD);
+  t.a1 = U(RH); t.a1T = U(RH); t.u2 = U(RH); t.u2T = U(RH); t.u1 = U(RH); t.u1T = U(RH);
+  t.dv1 = U(RH); t.dv1T = U(RH); t.dz2 = U(RH); t.dz2T = U(RH); t.dz1T = U(RH);
+  t.z1 = F(RH); t.s1 = F(RH); t.z2 = F(RH); t.a2 = F(RH); t.s2 = F(RH); t.v1 = F(RH); t.ds1 = F(RH);
+  t.du2 = F(RH); t.dz2f = F(RH); t.dz1f = F(RH);
+  t.f = F(rows); t.df = F(rows); t.e2 = F(rows);
+  t.lpart = F((s.Dp / 32) * rows);
+  t.rows = rows;
+}
+
 template <bool TA, bool TB>
 static void gemm(Surrogate& s, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                  int64_t ldc, int64_t M, int64_t N, int64_t K, float alpha, float beta) {
   HMC_REQUIRE(M % SG_T == 0 && N % SG_T == 0 && K % SG_K == 0, HMC_ERR_STATE, "surrogate GEMM padding");
   const dim3 grid((unsigned)(N / SG_T), (unsigned)(M / SG_T));
-  if (s.mode == 0)
-    hipLaunchKernelGGL((k_sgemm<TA, TB, true>), grid, dim3(256), 0, s.stream, A, lda, B, ldb, C, ldc,
-                       (int)K, alpha, beta);
-  else
-    hipLaunchKernelGGL((k_sgemm<TA, TB, false>), grid, dim3(256), 0, s.stream, A, lda, B, ldb, C, ldc,
-                       (int)K, alpha, beta);
+  hipLaunchKernelGGL((k_sgemm<TA, TB>), grid, dim3(256), 0, s.stream, A, lda, B, ldb, C, ldc, (int)K, alpha, beta);
   HMC_HIP(hipGetLastError());
 }
 
@@ -415,6 +1006,7 @@ static void ensure_planes(Surrogate& s, hipStream_t st) {
   hipLaunchKernelGGL(k_weight_plane, grid, dim3(256), 0, st, s.W2(), H, H, H, s.w2h, H, 0);
   hipLaunchKernelGGL(k_weight_plane, grid, dim3(256), 0, st, s.W2(), H, H, H, s.w2t, H, 1);
   HMC_HIP(hipGetLastError());
+  HMC_HIP(hipStreamSynchronize(st));   // later readers may be on another stream
   s.planes_ok = true;
 }
 
@@ -483,14 +1075,88 @@ static void backward(Surrogate& s, int64_t rows, float alpha, float beta) {
   HMC_HIP(hipGetLastError());
 }
 
-static void adam(Surrogate& s, float lr) {
+// the next Adam step (advances the step count)
+static AdamStep next_adam(Surrogate& s, float lr) {
   s.adam_t += 1;
-  s.planes_ok = false;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - std::pow(b1, (float)s.adam_t), c2 = 1.f - std::pow(b2, (float)s.adam_t);
-  hipLaunchKernelGGL(k_adam, g1(s.nP), dim3(256), 0, s.stream, s.P, s.dP, s.Pm, s.Pv, s.nP, lr, b1, b2, c1, c2,
-                     1e-8f);
+  return AdamStep{s.P, s.Pm, s.Pv, lr, b1, b2, c1, c2, 1e-8f};
+}
+
+static void adam(Surrogate& s, float lr) {
+  s.planes_ok = false;
+  hipLaunchKernelGGL(k_adam, g1(s.nP), dim3(256), 0, s.stream, next_adam(s, lr), s.dP, s.nP);
   HMC_HIP(hipGetLastError());
+}
+
+// ---- bf16 evaluation and training passes ------------------------------------
+template <class Epi>
+static void sur_gemm(Surrogate& s, int64_t M, int64_t N, const SurOperands& p0, const SurOperands& p1, const Epi& epi) {
+  // 32 x 32 tiles while there are few, with a second wave that only loads in a
+  // long product
+  auto go = [&](auto wm, auto wn, auto lw, auto st) {
+    constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value, LW = decltype(lw)::value, S = decltype(st)::value;
+    const int gm = (int)(M / (32 * WM)), gn = (int)(N / (32 * WN));
+    hipLaunchKernelGGL((k_sur_gemm<WM, WN, LW, S, Epi>), dim3((unsigned)((gm * gn + 7) / 8 * 8)),
+                       dim3((WM * WN + LW) * 64), 0, s.stream, p0, p1, gm, gn, epi);
+  };
+  using std::integral_constant;
+  using I0 = integral_constant<int, 0>;
+  using I1 = integral_constant<int, 1>;
+  using I2 = integral_constant<int, 2>;
+  if ((M / 32) * (N / 32) > 256) go(I2{}, I2{}, I0{}, integral_constant<int, 4>{});
+  else if (p0.K + p1.K <= 1024) go(I1{}, I1{}, I0{}, integral_constant<int, 8>{});
+  else go(I1{}, I1{}, I1{}, integral_constant<int, 9>{});
+  HMC_HIP(hipGetLastError());
+}
+
+// planes of rows idx of X (float32 [.][Dp]), forward to U1; f and (training) df
+static void bf16_forward(Surrogate& s, int64_t R, const float* X, const int32_t* idx, const float* y, float alpha,
+                         bool train) {
+  const int64_t H = s.H, Dp = s.Dp;
+  TrainBufs& t = s.tb;
+  hipLaunchKernelGGL(k_sur_rows, dim3((unsigned)(Dp / 64), (unsigned)(R / 64)), dim3(256), 0, s.stream, X, idx, Dp, R,
+                     t.x, train ? t.xT : nullptr);
+  HMC_HIP(hipGetLastError());
+  const SurOperands none{};
+  sur_gemm(s, R, H, SurOperands{t.x, s.w1h, Dp, Dp, (int)Dp}, none,
+           SurZ1{s.b1(), t.z1, t.s1, t.a1, train ? t.a1T : nullptr, H, R});                      // Z1 = Xn W1^T
+  sur_gemm(s, R, H, SurOperands{t.a1, s.w2h, H, H, (int)H}, none,
+           SurZ2{s.b2(), s.w3(), t.z2, t.a2, t.s2, t.u2, train ? t.u2T : nullptr, H, R});        // Z2 = A1 W2^T
+  hipLaunchKernelGGL(k_sur_head, dim3((unsigned)R), dim3(256), 0, s.stream, t.a2, s.w3(), s.b3(), y, idx, alpha, t.f,
+                     train ? t.df : nullptr, (int)H, (int)R);
+  sur_gemm(s, R, H, SurOperands{t.u2, s.w2t, H, H, (int)H}, none,
+           SurV1{t.s1, t.v1, t.u1, train ? t.u1T : nullptr, H, R});                              // V1 = U2 W2
+}
+
+// loss and parameter gradients (into dP), or with `step` the Adam update of
+// the parameters and of the weight planes
+static void bf16_train_batch(Surrogate& s, int64_t R, const float* X, const float* T, const float* y,
+                             const int32_t* idx, float alpha, float beta, const AdamStep* step, float* loss) {
+  const int64_t H = s.H, Dp = s.Dp;
+  TrainBufs& t = s.tb;
+  const SurOperands none{};
+  bf16_forward(s, R, X, idx, y, alpha, true);
+  sur_gemm(s, R, Dp, SurOperands{t.u1, s.w1t, H, H, (int)H}, none,
+           SurResid{T, idx, t.dg, t.dgT, t.lpart, s.D, Dp, R, beta});                            // G = U1 W1
+  sur_gemm(s, R, H, SurOperands{t.dg, s.w1h, Dp, Dp, (int)Dp}, none,
+           SurDU1{t.v1, t.s1, t.ds1, t.dv1, t.dv1T, H, R});                                      // dU1 = dG W1^T
+  sur_gemm(s, R, H, SurOperands{t.dv1, s.w2h, H, H, (int)H}, none,
+           SurDU2{s.w3(), t.z2, t.s2, t.df, t.du2, t.dz2f, t.dz2, t.dz2T, H, R});               // dU2 = dV1 W2^T
+  sur_gemm(s, R, H, SurOperands{t.dz2, s.w2t, H, H, (int)H}, none,
+           SurDA1{t.ds1, t.z1, t.s1, t.dz1f, t.dz1T, H, R});                                     // dA1 = dZ2 W2
+  const AdamStep ad = step ? *step : AdamStep{};
+  float* g = step ? nullptr : s.dP;
+  hipLaunchKernelGGL(k_sur_e2, dim3((unsigned)(R / 32)), dim3(256), 0, s.stream, t.lpart, (int)(Dp / 32), (int)R, t.e2);
+  hipLaunchKernelGGL(k_sur_finish, dim3((unsigned)(H / 64), 4), dim3(64), 0, s.stream,
+                     SurFinish{t.du2, t.s2, t.a2, t.dz2f, t.dz1f, t.e2, t.f, y, t.df, idx, g, ad, s.ow3, s.ob2, s.ob1,
+                               s.ob3, loss, (int)H, (int)R, (int)s.D, alpha, beta});
+  HMC_HIP(hipGetLastError());
+  // dW2 = U2^T dV1 + dZ2^T A1, dW1 = U1^T dG + dZ1^T Xn
+  sur_gemm(s, H, H, SurOperands{t.u2T, t.dv1T, R, R, (int)R}, SurOperands{t.dz2T, t.a1T, R, R, (int)R},
+           SurWeight{g, ad, s.oW2, s.w2h, s.w2t, H, H});
+  sur_gemm(s, H, Dp, SurOperands{t.u1T, t.dgT, R, R, (int)R}, SurOperands{t.dz1T, t.xT, R, R, (int)R},
+           SurWeight{g, ad, s.oW1, s.w1h, s.w1t, Dp, H});
 }
 
 // gradient of the surrogate at the chains' trajectory positions + kick/drift
@@ -695,22 +1361,38 @@ int hmc_surrogate_param_count(hmc_surrogate* h, int64_t* n) {
   });
 }
 
+// device allocations of one call
+struct FreeList {
+  std::vector<void*> v;
+  ~FreeList() {
+    for (void* p : v) (void)hipFree(p);
+  }
+};
+
 static void pack_unpack(Surrogate& s, float* host, bool to_device, float* dev) {
   // host layout is unpadded (W1 H x D); device rows are padded to Dp
+  if (!to_device) {
+    const int64_t np = s.H * s.D + s.nP - s.ob1;
+    if (s.D == s.Dp) {
+      d2h(host, dev, np * 4);
+      return;
+    }
+    FreeList tmp;   // packed on the device, one contiguous copy (a pitched copy runs row by row)
+    float* buf = (float*)dev_alloc(tmp.v, np * 4);
+    hipLaunchKernelGGL(k_sur_pack, dim3((unsigned)std::min<int64_t>((np + 255) / 256, 8192)), dim3(256), 0, s.stream,
+                       dev, s.H, s.D, s.Dp, np, buf);
+    HMC_HIP(hipGetLastError());
+    HMC_HIP(hipMemcpyAsync(host, buf, np * 4, hipMemcpyDeviceToHost, s.stream));
+    HMC_HIP(hipStreamSynchronize(s.stream));
+    return;
+  }
   std::vector<float> buf(s.nP, 0.f);
-  if (!to_device) d2h(buf.data(), dev, s.nP * 4);
   int64_t k = 0;
   for (int64_t r = 0; r < s.H; ++r)
-    for (int64_t c = 0; c < s.D; ++c, ++k) {
-      if (to_device) buf[s.oW1 + r * s.Dp + c] = host[k];
-      else host[k] = buf[s.oW1 + r * s.Dp + c];
-    }
+    for (int64_t c = 0; c < s.D; ++c, ++k) buf[s.oW1 + r * s.Dp + c] = host[k];
   const int64_t tail = s.nP - s.ob1;
-  for (int64_t i = 0; i < tail; ++i, ++k) {
-    if (to_device) buf[s.ob1 + i] = host[k];
-    else host[k] = buf[s.ob1 + i];
-  }
-  if (to_device) h2d(dev, buf.data(), s.nP * 4);
+  for (int64_t i = 0; i < tail; ++i, ++k) buf[s.ob1 + i] = host[k];
+  h2d(dev, buf.data(), s.nP * 4);
 }
 
 int hmc_surrogate_get_params(hmc_surrogate* h, float* params) {
@@ -733,35 +1415,73 @@ int hmc_surrogate_set_params(hmc_surrogate* h, const float* params) {
   });
 }
 
-// upload rows X (B x D, f64) normalised into s.Xn; returns padded row count
-static int64_t upload_norm(Surrogate& s, const double* X, int64_t B) {
-  const int64_t rows = round_up(B, 64);
-  ensure_rows(s, rows);
-  std::vector<float> hx(rows * s.Dp, 0.f), xm(s.Dp), xs(s.Dp);
-  d2h(xm.data(), s.xm, s.Dp * 4);
-  d2h(xs.data(), s.xs, s.Dp * 4);
-  for (int64_t b = 0; b < B; ++b)
-    for (int64_t j = 0; j < s.D; ++j) hx[b * s.Dp + j] = ((float)X[b * s.D + j] - xm[j]) / xs[j];
-  h2d(s.Xn, hx.data(), hx.size() * 4);
-  return rows;
+// rows (n x D, host f64) into float32 device rows dst [n][Dp] (k_sur_load's
+// mode), through a staging buffer of at most 64 MB
+static void load_rows(Surrogate& s, const double* rows, int64_t n, int mode, double fs, float* dst) {
+  const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(n, ((int64_t)64 << 20) / (8 * s.D)));
+  void* stage = nullptr;
+  if (hipMalloc(&stage, (size_t)chunk * s.D * 8) != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error{HMC_ERR_NOMEM, "surrogate staging buffer"};
+  }
+  try {
+    for (int64_t a = 0; a < n; a += chunk) {
+      const int64_t m = std::min(chunk, n - a);
+      HMC_HIP(hipMemcpyAsync(stage, rows + a * s.D, (size_t)m * s.D * 8, hipMemcpyHostToDevice, s.stream));
+      hipLaunchKernelGGL(k_sur_load, dim3((unsigned)std::min<int64_t>((m * s.Dp + 255) / 256, 8192)), dim3(256), 0,
+                         s.stream, (const double*)stage, m, s.D, s.Dp, s.xm, s.xs, fs, mode, dst + a * s.Dp);
+      HMC_HIP(hipGetLastError());
+    }
+    HMC_HIP(hipStreamSynchronize(s.stream));
+  } catch (...) {
+    (void)hipFree(stage);
+    throw;
+  }
+  (void)hipFree(stage);
+}
+
+// float32 device rows for a call: [rows][Dp], zero in the padding rows
+static float* call_rows(Surrogate& s, std::vector<void*>& tmp, int64_t rows) {
+  return (float*)dev_alloc(tmp, (size_t)rows * s.Dp * 4);
 }
 
 int hmc_surrogate_eval(hmc_surrogate* h, const double* X, int64_t B, double* f, double* g) {
   return guarded("hmc_surrogate_eval", [&] {
     HMC_REQUIRE(h && X && B > 0, HMC_ERR_ARG, "invalid argument");
     Surrogate& s = h->s;
-    const int64_t rows = upload_norm(s, X, B);
-    forward_grad(s, rows);
-    std::vector<float> hf(rows), hg(rows * s.Dp), gs(s.Dp);
-    HMC_HIP(hipMemcpyAsync(hf.data(), s.f, rows * 4, hipMemcpyDeviceToHost, s.stream));
-    HMC_HIP(hipMemcpyAsync(hg.data(), s.G, hg.size() * 4, hipMemcpyDeviceToHost, s.stream));
-    HMC_HIP(hipMemcpyAsync(gs.data(), s.gscale, s.Dp * 4, hipMemcpyDeviceToHost, s.stream));
-    HMC_HIP(hipStreamSynchronize(s.stream));
-    for (int64_t b = 0; b < B; ++b) {
-      if (f) f[b] = s.f_mean + s.f_scale * (double)hf[b];
+    const int64_t rows = round_up(B, 64);
+    std::vector<float> hf(rows);
+    FreeList tmp;
+    if (s.mode == 0) {
+      ensure_train_rows(s, rows);
+      ensure_planes(s, s.stream);
+      float* dx = call_rows(s, tmp.v, rows);
+      double* dg = g ? (double*)dev_alloc(tmp.v, (size_t)B * s.D * 8) : nullptr;
+      load_rows(s, X, B, 1, 1.0, dx);
+      bf16_forward(s, rows, dx, nullptr, nullptr, 0.f, false);
+      if (g) {
+        sur_gemm(s, rows, s.Dp, SurOperands{s.tb.u1, s.w1t, s.H, s.H, (int)s.H}, SurOperands{},
+                 SurEvalGrad{s.gscale, dg, s.D, B});
+        HMC_HIP(hipMemcpyAsync(g, dg, (size_t)B * s.D * 8, hipMemcpyDeviceToHost, s.stream));
+      }
+      HMC_HIP(hipMemcpyAsync(hf.data(), s.tb.f, rows * 4, hipMemcpyDeviceToHost, s.stream));
+      HMC_HIP(hipStreamSynchronize(s.stream));
+    } else {
+      ensure_rows(s, rows);
+      HMC_HIP(hipMemsetAsync(s.Xn, 0, (size_t)rows * s.Dp * 4, s.stream));
+      load_rows(s, X, B, 1, 1.0, s.Xn);
+      forward_grad(s, rows);
+      std::vector<float> hg(rows * s.Dp), gs(s.Dp);
+      HMC_HIP(hipMemcpyAsync(hf.data(), s.f, rows * 4, hipMemcpyDeviceToHost, s.stream));
+      HMC_HIP(hipMemcpyAsync(hg.data(), s.G, hg.size() * 4, hipMemcpyDeviceToHost, s.stream));
+      HMC_HIP(hipMemcpyAsync(gs.data(), s.gscale, s.Dp * 4, hipMemcpyDeviceToHost, s.stream));
+      HMC_HIP(hipStreamSynchronize(s.stream));
       if (g)
-        for (int64_t j = 0; j < s.D; ++j) g[b * s.D + j] = (double)hg[b * s.Dp + j] * (double)gs[j];
+        for (int64_t b = 0; b < B; ++b)
+          for (int64_t j = 0; j < s.D; ++j) g[b * s.D + j] = (double)hg[b * s.Dp + j] * (double)gs[j];
     }
+    if (f)
+      for (int64_t b = 0; b < B; ++b) f[b] = s.f_mean + s.f_scale * (double)hf[b];
   });
 }
 
@@ -772,22 +1492,28 @@ int hmc_surrogate_loss_grad(hmc_surrogate* h, const double* Xn, const double* y,
   return guarded("hmc_surrogate_loss_grad", [&] {
     HMC_REQUIRE(h && Xn && y && t && B > 0 && B % 64 == 0, HMC_ERR_ARG, "batch must be a positive multiple of 64");
     Surrogate& s = h->s;
-    ensure_rows(s, B);
-    std::vector<float> hx(B * s.Dp, 0.f), ht(B * s.Dp, 0.f), hy(B);
-    for (int64_t b = 0; b < B; ++b) {
-      hy[b] = (float)y[b];
-      for (int64_t j = 0; j < s.D; ++j) {
-        hx[b * s.Dp + j] = (float)Xn[b * s.D + j];
-        ht[b * s.Dp + j] = (float)t[b * s.D + j];
-      }
-    }
-    h2d(s.Xn, hx.data(), hx.size() * 4);
-    h2d(s.Tn, ht.data(), ht.size() * 4);
-    h2d(s.yb, hy.data(), B * 4);
-    forward_grad(s, B);
-    backward(s, B, (float)alpha, (float)beta);
+    std::vector<float> hy(B);
+    for (int64_t b = 0; b < B; ++b) hy[b] = (float)y[b];
+    FreeList tmp;
     float l = 0.f;
-    HMC_HIP(hipMemcpyAsync(&l, s.scal, 4, hipMemcpyDeviceToHost, s.stream));
+    if (s.mode == 0) {
+      ensure_train_rows(s, B);
+      ensure_planes(s, s.stream);
+      float *dx = call_rows(s, tmp.v, B), *dt = call_rows(s, tmp.v, B), *dy = (float*)dev_alloc(tmp.v, (B + 1) * 4);
+      h2d(dy, hy.data(), B * 4);
+      load_rows(s, Xn, B, 0, 1.0, dx);
+      load_rows(s, t, B, 0, 1.0, dt);
+      bf16_train_batch(s, B, dx, dt, dy, nullptr, (float)alpha, (float)beta, nullptr, dy + B);
+      HMC_HIP(hipMemcpyAsync(&l, dy + B, 4, hipMemcpyDeviceToHost, s.stream));
+    } else {
+      ensure_rows(s, B);
+      h2d(s.yb, hy.data(), B * 4);
+      load_rows(s, Xn, B, 0, 1.0, s.Xn);
+      load_rows(s, t, B, 0, 1.0, s.Tn);
+      forward_grad(s, B);
+      backward(s, B, (float)alpha, (float)beta);
+      HMC_HIP(hipMemcpyAsync(&l, s.scal, 4, hipMemcpyDeviceToHost, s.stream));
+    }
     HMC_HIP(hipStreamSynchronize(s.stream));
     if (loss) *loss = (double)l / (double)B;
     if (grad) pack_unpack(s, grad, false, s.dP);
@@ -803,53 +1529,49 @@ int hmc_surrogate_train(hmc_surrogate* h, const double* X, const double* chi, co
     HMC_REQUIRE(h && X && chi && grad && N >= batch && batch > 0 && batch % 64 == 0 && epochs > 0, HMC_ERR_ARG,
                 "invalid training arguments");
     Surrogate& s = h->s;
-    ensure_rows(s, batch);
+    const int64_t nb = N / batch;
+    if (s.mode == 0) {
+      ensure_train_rows(s, batch);
+      ensure_planes(s, s.stream);
+    } else {
+      ensure_rows(s, batch);
+    }
     // normalised training set on the device
-    std::vector<float> xm(s.Dp), xs(s.Dp);
-    d2h(xm.data(), s.xm, s.Dp * 4);
-    d2h(xs.data(), s.xs, s.Dp * 4);
-    std::vector<void*> tmp;
-    float* dX = (float*)dev_alloc(tmp, (size_t)N * s.Dp * 4);
-    float* dT = (float*)dev_alloc(tmp, (size_t)N * s.Dp * 4);
-    float* dy = (float*)dev_alloc(tmp, (size_t)N * 4);
-    try {
-      std::vector<float> hx((size_t)N * s.Dp, 0.f), ht((size_t)N * s.Dp, 0.f), hy(N);
-      for (int64_t i = 0; i < N; ++i) {
-        for (int64_t j = 0; j < s.D; ++j) {
-          hx[i * s.Dp + j] = (float)((X[i * s.D + j] - xm[j]) / xs[j]);
-          ht[i * s.Dp + j] = (float)(grad[i * s.D + j] * xs[j] / s.f_scale);   // d f_n / d x_n
-        }
-        hy[i] = (float)((chi[i] - s.f_mean) / s.f_scale);
-      }
-      h2d(dX, hx.data(), hx.size() * 4);
-      h2d(dT, ht.data(), ht.size() * 4);
-      h2d(dy, hy.data(), N * 4);
-      std::vector<int32_t> perm(N);
-      std::iota(perm.begin(), perm.end(), 0);
-      std::mt19937_64 g(seed);
-      const int64_t nb = N / batch;
-      for (int64_t e = 0; e < epochs; ++e) {
-        std::shuffle(perm.begin(), perm.end(), g);
-        double acc = 0.0;
-        for (int64_t b = 0; b < nb; ++b) {
-          HMC_HIP(hipMemcpyAsync(s.idx, perm.data() + b * batch, batch * 4, hipMemcpyHostToDevice, s.stream));
-          hipLaunchKernelGGL(k_gather, g1(batch * s.Dp), dim3(256), 0, s.stream, dX, dT, dy, s.idx, s.Xn, s.Tn,
-                             s.yb, s.Dp, batch);
+    FreeList tmp;
+    float *dX = call_rows(s, tmp.v, N), *dT = call_rows(s, tmp.v, N), *dy = (float*)dev_alloc(tmp.v, (size_t)N * 4);
+    int32_t* idx = (int32_t*)dev_alloc(tmp.v, (size_t)N * 4);
+    float* dl = (float*)dev_alloc(tmp.v, (size_t)nb * 4);
+    std::vector<float> hy(N), hl(nb);
+    for (int64_t i = 0; i < N; ++i) hy[i] = (float)((chi[i] - s.f_mean) / s.f_scale);
+    h2d(dy, hy.data(), N * 4);
+    load_rows(s, X, N, 2, 1.0, dX);
+    load_rows(s, grad, N, 3, s.f_scale, dT);   // d f_n / d x_n
+    std::vector<int32_t> perm(N);
+    std::iota(perm.begin(), perm.end(), 0);
+    std::mt19937_64 g(seed);
+    for (int64_t e = 0; e < epochs; ++e) {
+      std::shuffle(perm.begin(), perm.end(), g);
+      HMC_HIP(hipMemcpyAsync(idx, perm.data(), N * 4, hipMemcpyHostToDevice, s.stream));
+      HMC_HIP(hipStreamSynchronize(s.stream));   // perm is shuffled again while the epoch runs
+      for (int64_t b = 0; b < nb; ++b) {
+        if (s.mode == 0) {
+          const AdamStep step = next_adam(s, (float)lr);   // updates the planes too
+          bf16_train_batch(s, batch, dX, dT, dy, idx + b * batch, (float)alpha, (float)beta, &step, dl + b);
+        } else {
+          hipLaunchKernelGGL(k_gather, g1(batch * s.Dp), dim3(256), 0, s.stream, dX, dT, dy, idx + b * batch, s.Xn,
+                             s.Tn, s.yb, s.Dp, batch);
           forward_grad(s, batch);
           backward(s, batch, (float)alpha, (float)beta);
           adam(s, (float)lr);
-          float l = 0.f;
-          HMC_HIP(hipMemcpyAsync(&l, s.scal, 4, hipMemcpyDeviceToHost, s.stream));
-          HMC_HIP(hipStreamSynchronize(s.stream));
-          acc += (double)l / (double)batch;
+          HMC_HIP(hipMemcpyAsync(dl + b, s.scal, 4, hipMemcpyDeviceToDevice, s.stream));
         }
-        if (loss_history) loss_history[e] = acc / (double)nb;
       }
-    } catch (...) {
-      for (void* p : tmp) (void)hipFree(p);
-      throw;
+      HMC_HIP(hipMemcpyAsync(hl.data(), dl, nb * 4, hipMemcpyDeviceToHost, s.stream));
+      HMC_HIP(hipStreamSynchronize(s.stream));
+      double acc = 0.0;
+      for (int64_t b = 0; b < nb; ++b) acc += (double)hl[b] / (double)batch;
+      if (loss_history) loss_history[e] = acc / (double)nb;
     }
-    for (void* p : tmp) (void)hipFree(p);
   });
 }
 
