@@ -1011,7 +1011,26 @@ int hmc_chains_run(hmc_chains* hc, int64_t proposals, int L, int integrator, dou
     HMC_HIP(hipMemcpyAsync(c.step, stepsize, c.B * 8, hipMemcpyHostToDevice, P.stream));
     HMC_HIP(hipMemsetAsync(c.acc_count, 0, c.B * 8, P.stream));
     const bool gemm = P.resolved_engine() == HMC_ENGINE_GEMM;
-    for (int64_t i = 0; i < proposals; ++i) {
+    int64_t done = 0;
+    if (!gemm && fused_runs_many(c) && proposals > 0) {
+      // all proposals, or those before one whose trace or history slot is
+      // missing (which the loop below then reports)
+      const int64_t slot0 = c.tr_cap > 0 ? c.tr_n : -1;
+      const int64_t hist0 = autotune && c.hist_cap > 0 ? c.hist_n : -1;
+      int64_t tr = c.tr_n, hist = c.hist_n;
+      for (; done < proposals; ++done) {
+        const bool rec = slot0 >= 0 && (first_proposal + done) % thinning == 0;
+        if ((rec && tr >= c.tr_cap) || (hist0 >= 0 && hist >= c.hist_cap)) break;
+        tr += rec;
+        hist += hist0 >= 0;
+      }
+      if (done > 0)
+        fused_run(c, done, L, integrator, seed, first_proposal, randomize, autotune, target, learning_rate, thinning,
+                  slot0, hist0);
+      c.tr_n = tr;
+      c.hist_n = hist;
+    }
+    for (int64_t i = done; i < proposals; ++i) {
       const int64_t prop = first_proposal + i;
       int64_t slot = -1;
       if (c.tr_cap > 0 && prop % thinning == 0) {

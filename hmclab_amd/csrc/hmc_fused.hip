@@ -674,6 +674,401 @@ __global__ __launch_bounds__((fu_nt<T, SPARSE>())) void k_fused_propose(Ops<T, V
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small dense targets in float64: whole proposals, several in one launch.  One
+// workgroup carries CT chains; thread t owns parameter t (position, momentum and
+// model constants in registers for the whole launch).  A product row is cut into
+// k parts over the waves: with S = ceil(rows / 64) row slices and fewer slices
+// than waves, wave w sums part w / S of slice w % S and the parts are added in a
+// fixed order, so every wave works and a stage's chain of loads is row length /
+// parts long.  The order of the sums depends on the sizes alone.
+//
+// What bounds it: latency (loads, LDS, barriers) on one CU per tile of chains.
+// With premultiplied trajectories and at most RK columns per part the thread's
+// piece of H stays in registers, and a stage touches no memory but LDS: 0.51 us
+// at 100 x 50 against 1.57 us in k_fused_propose, whose rows are one thread's
+// chain of loads; the rest of a proposal 4.0 us against 10 us (one launch for
+// many proposals, momenta drawn for several proposals by as many waves).
+// ---------------------------------------------------------------------------
+struct DenseRun {
+  const double *H, *hb;      // premultiplied trajectories (k-major view), or null
+  const double *Gt, *G;      // k-major views of the forward and backward operators
+  int64_t ldh, ldgt, ldg;
+  int n, d;
+  int count;                 // proposals of this launch
+  int64_t thinning;          // trace slots: proposals with index % thinning == 0
+  int64_t slot0, hist0;      // first trace / tuning history slot (or -1)
+};
+
+constexpr int DR_U = 16;     // matrix loads in flight per lane
+constexpr int DR_NT = 512, DR_NW = DR_NT / 64;
+constexpr int DR_MAX_D = 192;   // parameters (see dense_plan)
+
+// Sums over k-major rows (element (row, k) at M[k * ld + row]) of in[k][CT].
+// With one part each lane calls f(row, acc); otherwise the parts go to
+// part[p][row][CT] and the caller adds them after a barrier.
+template <int CT, int NW>
+struct DensePass {
+  const double* M;
+  uint32_t ld8;        // bytes between consecutive k (an operator is below 4 GB)
+  int rows, K, S, parts;
+  int u, k0, k1;       // the wave's unit (slice + S * part) and k range; idle: u < 0
+  __device__ __forceinline__ DensePass(const double* m, int64_t ld, int rows_, int K_, int w)
+      : M(m), ld8((uint32_t)ld * 8u), rows(rows_), K(K_) {
+    S = (rows + 63) / 64;
+    parts = S < NW ? NW / S : 1;
+    u = w < S * parts ? w : -1;
+    const int p = w / S;
+    k0 = parts > 1 ? p * K / parts : 0;
+    k1 = parts > 1 ? (p + 1) * K / parts : K;
+  }
+  __device__ __forceinline__ void dot(int row, const double* in, double (&acc)[CT]) const {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[c] = 0.0;
+    const char* base = reinterpret_cast<const char*>(M);
+    uint32_t off = (uint32_t)(row < rows ? row : rows - 1) * 8u + (uint32_t)k0 * ld8;
+    int k = k0;
+    for (; k + DR_U <= k1; k += DR_U) {
+      double v[DR_U];
+#pragma unroll
+      for (int i = 0; i < DR_U; ++i, off += ld8) v[i] = *reinterpret_cast<const double*>(base + off);
+#pragma unroll
+      for (int i = 0; i < DR_U; ++i)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c] += v[i] * in[(k + i) * CT + c];
+    }
+    // remainder by halves, so that its loads are in flight together as well
+#pragma unroll
+    for (int h = DR_U / 2; h >= 1; h /= 2) {
+      if (k1 - k >= h) {
+        double v[DR_U / 2];
+#pragma unroll
+        for (int i = 0; i < h; ++i, off += ld8) v[i] = *reinterpret_cast<const double*>(base + off);
+#pragma unroll
+        for (int i = 0; i < h; ++i)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[c] += v[i] * in[(k + i) * CT + c];
+        k += h;
+      }
+    }
+  }
+  template <class F>
+  __device__ __forceinline__ void run(const double* in, double* part, int lane, F&& f) const {
+    if (parts > 1) {
+      if (u < 0) return;
+      double acc[CT];
+      const int s = u % S;
+      dot(s * 64 + lane, in, acc);
+#pragma unroll
+      for (int c = 0; c < CT; ++c) part[(u * 64 + lane) * CT + c] = acc[c];   // u = s + S p
+      return;
+    }
+    for (int s = u; s >= 0 && s < S; s += NW) {
+      double acc[CT];
+      const int row = s * 64 + lane;
+      dot(row, in, acc);
+      if (row < rows) f(row, acc);
+    }
+  }
+  // sum of a row's parts: all loads at once, then a fixed tree
+  __device__ __forceinline__ double sum(const double* part, int row, int c) const {
+    double v[NW];
+#pragma unroll
+    for (int p = 0; p < NW; ++p) v[p] = p < parts ? part[(p * S * 64 + row) * CT + c] : 0.0;
+#pragma unroll
+    for (int h = NW / 2; h >= 1; h /= 2)
+#pragma unroll
+      for (int p = 0; p < h; ++p) v[p] += v[p + h];
+    return v[0];
+  }
+};
+
+// Block-wide sums of V doubles per thread, returned to every thread: butterflies
+// inside the waves, one LDS pass, then 16 lanes per value
+template <int V, int NW>
+__device__ inline void block_sums(double (&v)[V], double* red) {
+  static_assert(NW <= 16, "one 16-lane group per value");
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < V; ++i) v[i] += __shfl_xor(v[i], off, 64);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) red[i * 16 + w] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i0 = 0; i0 < V; i0 += 4) {
+    const int i = i0 + (lane >> 4), l = lane & 15;
+    double t = (i < V && l < NW) ? red[i * 16 + l] : 0.0;
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) t += __shfl_xor(t, off, 64);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (i0 + g < V) v[i0 + g] = __shfl(t, 16 * g, 64);
+  }
+}
+
+template <int CT, int RK, bool PM>
+__global__ __launch_bounds__(DR_NT) void k_dense_run(DenseRun q, FusedArgs a, DevModel md) {
+  constexpr int NT = DR_NT, NW = DR_NW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int n = q.n, d = q.d;
+  double* Xs = reinterpret_cast<double*>(smem_raw);   // [d + RK][CT], zero past d
+  double* part = Xs + (d + RK) * CT;                  // [NW * 64][CT]
+  double* zs = part + NW * 64 * CT;                   // [groups][d][CT] momenta of the next proposals
+  // momenta are drawn for `groups` proposals at a time, 64 S threads each: a
+  // draw is a long chain of operations, and most threads own no parameter
+  const int groups = NT / (64 * ((d + 63) / 64));
+  double* Rs = zs + groups * d * CT;                  // [n][CT] (residual form)
+  __shared__ double red[3 * CT * 16], s_step[CT];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t c0 = (int64_t)blockIdx.x * CT;
+  const bool own = tid < d;
+  const int j = own ? tid : 0;
+  double* x0 = reinterpret_cast<double*>(a.x0);
+  const ParamCst<double> pc = param_cst<double>(md, j);
+  auto kin = [&](double pv) { return md.minv ? pv * (pc.minv * pv) : pv * pv; };   // as kterm
+  const double my_dobs = tid < n ? a.dobs[tid] : 0.0, my_var = tid < n ? a.var[tid] : 1.0;
+
+  // gradient product (H, or the backward operator) and forward product
+  const DensePass<CT, NW> hp(PM ? q.H : q.G, PM ? q.ldh : q.ldg, d, PM ? d : n, w), fp(q.Gt, q.ldgt, n > 0 ? n : 1, d, w);
+  // this thread's piece of H (RK > 0): the k range of its wave
+  double hreg[RK > 0 ? RK : 1];
+  if constexpr (RK > 0) {
+    const int row = (hp.u >= 0 ? hp.u % hp.S : 0) * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < RK; ++i)
+      hreg[i] = (hp.u >= 0 && row < d && hp.k0 + i < hp.k1) ? q.H[(int64_t)(hp.k0 + i) * q.ldh + row] : 0.0;
+    for (int i = tid; i < RK * CT; i += NT) Xs[d * CT + i] = 0.0;
+  }
+  const double hbj = (PM && own) ? q.hb[j] : 0.0;
+
+  double xc[CT], chi[CT], beta[CT];   // current positions and misfits
+  int64_t accepted[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const bool on = c0 + c < a.B;
+    xc[c] = (on && own) ? x0[(c0 + c) * a.ldx + j] : 0.0;
+    chi[c] = on ? a.chi0[c0 + c] : 0.0;
+    beta[c] = (on && a.beta) ? a.beta[c0 + c] : 1.0;
+    accepted[c] = 0;
+  }
+  if (tid < CT) s_step[tid] = (a.step && c0 + tid < a.B) ? a.step[c0 + tid] : 0.0;
+  __syncthreads();
+
+  int64_t slot = q.slot0, hist = q.hist0;
+  for (int it = 0; it < q.count; ++it) {
+    const int64_t prop = a.prop + it;
+    // sums over the block: K0, misfit (infinite out of bounds), K1
+    double e[CT], ua[CT], x[CT], p[CT], sums[3 * CT];
+#pragma unroll
+    for (int i = 0; i < 3 * CT; ++i) sums[i] = 0.0;
+    if (!a.p_host && it % groups == 0) {
+      const int span = 64 * ((d + 63) / 64), gi = tid / span, jj = tid - gi * span;
+      if (gi < groups && jj < d && it + gi < q.count) {
+        const double mj = md.msqrt ? md.msqrt[jj] : 1.0;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          double z0, z1;
+          philox_normal2(a.seed, (uint32_t)(c0 + c < a.B ? c0 + c : a.B - 1), (uint64_t)(prop + gi),
+                         (uint32_t)(jj >> 1), z0, z1);
+          zs[(gi * d + jj) * CT + c] = mj * ((jj & 1) ? z1 : z0);
+        }
+      }
+      __syncthreads();
+    }
+    // ---- step, momentum, first drift
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int64_t ch = c0 + c < a.B ? c0 + c : a.B - 1;
+      if (a.device_scalars) {
+        double ue;
+        philox_scalars(a.seed, (uint32_t)ch, (uint64_t)prop, ue, ua[c]);
+        e[c] = a.randomize ? ue * s_step[c] : s_step[c];
+      } else {
+        e[c] = a.eps[ch];
+        ua[c] = a.u[ch];
+      }
+      x[c] = xc[c];
+      p[c] = 0.0;
+      if (own) {
+        p[c] = a.p_host ? a.p_host[ch * a.ldx + j] : zs[((it % groups) * d + j) * CT + c];
+        sums[c] = kin(p[c]);
+        x[c] += (a.first_drift * e[c]) * (pc.minv * p[c]);
+        corrector_c<double>(pc, x[c], p[c]);
+        Xs[j * CT + c] = x[c];
+      }
+    }
+    __syncthreads();
+
+    // ---- stages: gradient, kick, drift (+ drift2)
+    for (int step = 0, k = 0; step < a.L; k = k + 1 < a.P ? k + 1 : (++step, 0)) {
+      const double* sc = (step + 1 < a.L) ? a.pat[k] : a.pat_last[k];
+      const double kick = sc[0], drift = sc[1], drift2 = sc[2];
+      double g[CT];
+      if constexpr (RK > 0) {
+        if (hp.u >= 0) {
+          double acc[CT];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[c] = 0.0;
+#pragma unroll
+          for (int i = 0; i < RK; ++i)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[c] += hreg[i] * Xs[(hp.k0 + i) * CT + c];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) part[tid * CT + c] = acc[c];   // u * 64 + lane
+        }
+        __syncthreads();
+      } else {
+        if (!PM && n > 0) {
+          fp.run(Xs, part, lane, [&](int i, double* acc) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) Rs[i * CT + c] = (acc[c] - a.dobs[i]) / a.var[i];
+          });
+          __syncthreads();
+          if (fp.parts > 1) {
+            if (tid < n) {
+#pragma unroll
+              for (int c = 0; c < CT; ++c) Rs[tid * CT + c] = (fp.sum(part, tid, c) - my_dobs) / my_var;
+            }
+            __syncthreads();
+          }
+        }
+        if (PM || n > 0) {
+          hp.run(PM ? Xs : Rs, part, lane, [&](int row, double* acc) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) part[row * CT + c] = acc[c];
+          });
+          __syncthreads();
+        }
+      }
+      if (own) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) g[c] = (PM || n > 0) ? hp.sum(part, j, c) - hbj : 0.0;
+      }
+      if (own) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          double gg = g[c] + prior_grad_c<double>(md, pc, x[c]);
+          if (x[c] < pc.lo || x[c] > pc.hi) gg = INFINITY;
+          p[c] -= (a.beta ? kick * e[c] * beta[c] : kick * e[c]) * gg;
+          x[c] += (drift * e[c]) * (pc.minv * p[c]);
+          corrector_c<double>(pc, x[c], p[c]);
+          if (drift2 != 0.0) {
+            x[c] += (drift2 * e[c]) * (pc.minv * p[c]);
+            corrector_c<double>(pc, x[c], p[c]);
+          }
+          Xs[j * CT + c] = x[c];
+        }
+      }
+      __syncthreads();
+    }
+
+    // ---- endpoint: data misfit, prior, bounds, kinetic energy
+    if (n > 0) {
+      auto add = [&](double dv, double vv, const double* acc) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          const double rr = acc[c] - dv;
+          sums[CT + c] += 0.5 * (rr * rr / vv);
+        }
+      };
+      fp.run(Xs, part, lane, [&](int i, double* acc) { add(a.dobs[i], a.var[i], acc); });
+      if (fp.parts > 1) {
+        __syncthreads();
+        if (tid < n) {
+          double acc[CT];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[c] = fp.sum(part, tid, c);
+          add(my_dobs, my_var, acc);
+        }
+      }
+    }
+    if (own) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        double pm = 0.0;
+#pragma unroll
+        for (int k = 0; k < kMaxPriors; ++k) {
+          if (k >= md.n_priors) break;
+          if (md.pr[k].kind == HMC_PRIOR_NORMAL) {
+            const double r = pc.a[k] - x[c];
+            pm += 0.5 * (r * (pc.b[k] * r));
+          } else {
+            pm += fabs(x[c] - pc.a[k]) * pc.b[k];
+          }
+        }
+        sums[CT + c] += (x[c] < pc.lo || x[c] > pc.hi) ? INFINITY : pm;
+        sums[2 * CT + c] = kin(p[c]);
+      }
+    }
+    block_sums<3 * CT, NW>(sums, red);
+
+    // ---- Metropolis: every thread takes the same decision
+    const bool rec = slot >= 0 && prop % q.thinning == 0;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int64_t ch = c0 + c;
+      const double chi1 = sums[CT + c] + a.mconst;
+      const double H0 = beta[c] * chi[c] + 0.5 * sums[c];
+      const double H1 = beta[c] * chi1 + 0.5 * sums[2 * CT + c];
+      const double av = exp(H0 - H1);
+      const bool ok = av > ua[c];
+      if (ok) {
+        chi[c] = chi1;
+        xc[c] = x[c];
+        accepted[c] += 1;
+      }
+      if (ch < a.B) {
+        if (tid == 0) {
+          if (a.autotune) {
+            if (hist >= 0) {
+              a.hist_rate[hist * a.B + ch] = av;
+              a.hist_step[hist * a.B + ch] = s_step[c];
+            }
+            const double wgt = pow((double)(prop + 1), -a.lr);
+            const double ar = isnan(av) ? 0.0 : av;
+            double sv = s_step[c] - wgt * (a.target - fmin(ar, 1.0));
+            if (sv <= 0.0) sv = fmax(sv, 1e-18);
+            s_step[c] = sv;
+          }
+          if (it + 1 == q.count) {
+            if (a.device_scalars) {
+              a.eps[ch] = e[c];
+              a.u[ch] = ua[c];
+            }
+            if (a.h0) a.h0[ch] = H0;
+            if (a.h1) a.h1[ch] = H1;
+            if (a.acc) a.acc[ch] = ok ? 1 : 0;
+          }
+          if (rec) a.tr_chi[slot * a.B + ch] = beta[c] * chi[c];
+        }
+        if (own) {
+          if (rec) reinterpret_cast<double*>(a.tr_x)[(slot * a.B + ch) * d + j] = xc[c];
+          if (a.x_out) reinterpret_cast<double*>(a.x_out)[ch * a.ldx + j] = x[c];
+          if (a.p_out) reinterpret_cast<double*>(a.p_out)[ch * a.ldx + j] = p[c];
+        }
+      }
+    }
+    if (rec) ++slot;
+    if (hist >= 0) ++hist;
+    __syncthreads();   // the sums and steps of this proposal have been read
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const int64_t ch = c0 + c;
+    if (ch >= a.B) continue;
+    if (own) x0[ch * a.ldx + j] = xc[c];
+    if (tid == 0) {
+      a.chi0[ch] = chi[c];
+      if (a.acc_count) a.acc_count[ch] += accepted[c];
+      if (a.autotune) a.step[ch] = s_step[c];
+    }
+  }
+}
+
 // misfit (FP64) and gradient (trajectory precision) of model rows
 template <typename T, typename VT, bool SPARSE, int CT, int KMAX>
 __global__ __launch_bounds__((fu_nt<T, SPARSE>())) void k_fused_eval(Ops<T, VT, SPARSE> op, const T* X, int64_t ldx,
@@ -992,21 +1387,14 @@ static void dispatch(const Problem& p, int ct, int kmax, F&& f) {
   }
 }
 
-void fused_propose(Chains& c, bool host_p, int L, int integrator, uint64_t seed, int64_t prop,
-                   int randomize, int autotune, double target, double learning_rate,
-                   int64_t trace_slot, int64_t hist_slot) {
+// arguments of `prop`-th proposal(s); trace and history slots of the first
+static FusedArgs fused_args(Chains& c, bool host_p, int L, int integrator, uint64_t seed, int64_t prop, int randomize,
+                            int autotune, double target, double learning_rate, int64_t trace_slot, int64_t hist_slot) {
   Problem& p = *c.p;
-  size_t lds = 0;
-  const int ct = fused_ct(p, c.B, lds);
-  const int kmax = fused_kmax(p);
   double first = 0.0;
   std::vector<Stage> st;
   integrator_schedule(integrator, L, first, st);
   const int P = (int)st.size() / L;
-  if (trace_slot >= 0) HMC_REQUIRE(trace_slot < c.tr_cap, HMC_ERR_STATE, "trace capacity exceeded");
-  if (hist_slot >= 0) HMC_REQUIRE(hist_slot < c.hist_cap, HMC_ERR_STATE, "tuning history capacity exceeded");
-  fused_premult_build(c);
-
   FusedArgs a{};
   a.x0 = c.x0;
   a.chi0 = c.chi0;
@@ -1048,6 +1436,136 @@ void fused_propose(Chains& c, bool host_p, int L, int integrator, uint64_t seed,
     a.pat[k][0] = s0.kick; a.pat[k][1] = s0.drift; a.pat[k][2] = s0.drift2;
     a.pat_last[k][0] = s1.kick; a.pat_last[k][1] = s1.drift; a.pat_last[k][2] = s1.drift2;
   }
+  return a;
+}
+
+// ---- small dense float64 targets: k_dense_run ---------------------------------
+// LDS bytes of a launch with ct chains (rk: columns of H a thread holds)
+static size_t dense_run_lds(const Problem& p, bool premult, int ct, int rk) {
+  const size_t groups = DR_NT / (64 * ((p.d + 63) / 64));
+  return ((size_t)(p.d + rk) + (size_t)DR_NT + groups * p.d + (premult ? 0 : (size_t)p.n)) * ct * 8;
+}
+
+struct DensePlan {
+  int ct = 0, rk = 0;
+};
+
+// Chains per workgroup: one while that gives every CU at most one workgroup,
+// else two, which share the matrix loads; ct 0: k_fused_propose takes the
+// problem.  Up to 192 parameters a row's sum is cut into at least two parts
+// that leave a wave's piece of the operator short; beyond, a stage is bound by
+// streaming the operator from L2 (about 60 GB/s per CU) in either kernel, and two
+// chains per workgroup lose what one launch per proposal saved.  L = 10, us per
+// proposal here and there: one to four chains, 100 x 50 9.0 / 25.8, 220 x 120
+// 16 / 44, 300 x 160 51 / 64, 300 x 190 58 / 68, 400 x 250 95 / 104; 512 chains,
+// 90 x 60 16 / 39, 60 x 130 55 / 77, 200 x 190 69 / 79, 400 x 192 72 / 78,
+// 400 x 250 108 / 105, 200 x 250 176 / 164.  Problems and tiles that fused_ct
+// refuses are refused here as well.
+static DensePlan dense_plan(const Problem& p, int64_t B) {
+  DensePlan pl;
+  if (p.op == 2 || p.state_dtype != HMC_F64 || p.d > DR_MAX_D) return pl;
+  size_t lds = 0;
+  fused_ct(p, B, lds);
+  int dev = 0, n_cu = 256;
+  HMC_HIP(hipGetDevice(&dev));
+  HMC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+  const bool pm = fused_premult(p);
+  const int slices = (int)((p.d + 63) / 64), parts = DR_NW / slices;
+  const int kmax = (int)((p.d + parts - 1) / parts);
+  pl.rk = !pm ? 0 : kmax <= 8 ? 8 : kmax <= 16 ? 16 : kmax <= 32 ? 32 : 0;
+  pl.ct = p.fused_ct > 0 ? p.fused_ct : B <= n_cu ? 1 : 2;
+  const size_t budget = 160 * 1024 - 4096;
+  while (pl.ct > 0 && dense_run_lds(p, pm, pl.ct, pl.rk) > budget) pl.ct = p.fused_ct > 0 ? 0 : pl.ct - 1;
+  return pl;
+}
+
+static void launch_dense(Chains& c, const DensePlan& pl, const FusedArgs& a, int count, int64_t thinning,
+                         int64_t slot0, int64_t hist0) {
+  Problem& p = *c.p;
+  DenseRun q{};
+  const bool pm = fused_premult(p);
+  if (pm) {
+    q.H = p.H;
+    q.hb = p.hb;
+    q.ldh = p.ldh;
+  }
+  q.Gt = (const double*)p.Gt_tgt;
+  q.G = (const double*)p.G;
+  q.ldgt = p.ldgt;
+  q.ldg = p.ldg;
+  q.n = (int)p.n;
+  q.d = (int)p.d;
+  q.count = count;
+  q.thinning = thinning;
+  q.slot0 = slot0;
+  q.hist0 = hist0;
+  const size_t lds = dense_run_lds(p, pm, pl.ct, pl.rk);
+  const dim3 grid((unsigned)((c.B + pl.ct - 1) / pl.ct));
+  const DevModel md = p.model();
+  auto go = [&](auto ct, auto rk, auto form) {
+    auto kern = k_dense_run<decltype(ct)::value, decltype(rk)::value, decltype(form)::value>;
+    if (lds > 65536)
+      HMC_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, grid, dim3(DR_NT), lds, p.stream, q, a, md);
+  };
+  using std::integral_constant;
+  auto by_ct = [&](auto rk, auto form) {
+    if (pl.ct == 2) go(integral_constant<int, 2>{}, rk, form);
+    else go(integral_constant<int, 1>{}, rk, form);
+  };
+  using PM = std::true_type;
+  if (!pm) by_ct(integral_constant<int, 0>{}, std::false_type{});
+  else if (pl.rk == 8) by_ct(integral_constant<int, 8>{}, PM{});
+  else if (pl.rk == 16) by_ct(integral_constant<int, 16>{}, PM{});
+  else if (pl.rk == 32) by_ct(integral_constant<int, 32>{}, PM{});
+  else by_ct(integral_constant<int, 0>{}, PM{});
+  HMC_HIP(hipGetLastError());
+}
+
+bool fused_runs_many(const Chains& c) {
+  return !c.timing && !c.ex_pairs && dense_plan(*c.p, c.B).ct > 0;
+}
+
+// `count` consecutive device-RNG proposals; the first trace slot (-1: no trace)
+// takes the first proposal whose index is a multiple of thinning
+void fused_run(Chains& c, int64_t count, int L, int integrator, uint64_t seed, int64_t prop, int randomize,
+               int autotune, double target, double learning_rate, int64_t thinning, int64_t slot0, int64_t hist0) {
+  fused_premult_build(c);
+  const DensePlan pl = dense_plan(*c.p, c.B);
+  FusedArgs a = fused_args(c, false, L, integrator, seed, prop, randomize, autotune, target, learning_rate, slot0, hist0);
+  // bounded launches: about 20000 stages each
+  const int64_t most = std::max<int64_t>(1, 20000 / ((int64_t)a.L * a.P));
+  for (int64_t i = 0; i < count;) {
+    const int64_t m = std::min(most, count - i);
+    a.prop = prop + i;
+    launch_dense(c, pl, a, (int)m, thinning, slot0, hist0);
+    if (slot0 >= 0)
+      for (int64_t k = prop + i; k < prop + i + m; ++k) slot0 += k % thinning == 0;
+    if (hist0 >= 0) hist0 += m;
+    i += m;
+  }
+}
+
+void fused_propose(Chains& c, bool host_p, int L, int integrator, uint64_t seed, int64_t prop,
+                   int randomize, int autotune, double target, double learning_rate,
+                   int64_t trace_slot, int64_t hist_slot) {
+  Problem& p = *c.p;
+  if (trace_slot >= 0) HMC_REQUIRE(trace_slot < c.tr_cap, HMC_ERR_STATE, "trace capacity exceeded");
+  if (hist_slot >= 0) HMC_REQUIRE(hist_slot < c.hist_cap, HMC_ERR_STATE, "tuning history capacity exceeded");
+  fused_premult_build(c);
+  const FusedArgs a = fused_args(c, host_p, L, integrator, seed, prop, randomize, autotune, target, learning_rate,
+                                 trace_slot, hist_slot);
+  const DensePlan pl = dense_plan(p, c.B);
+  if (pl.ct > 0) {
+    hipEvent_t ev;
+    time_begin(c, 0, ev);
+    launch_dense(c, pl, a, 1, 1, trace_slot, hist_slot);
+    time_end(c, 0, ev);
+    return;
+  }
+  size_t lds = 0;
+  const int ct = fused_ct(p, c.B, lds);
+  const int kmax = fused_kmax(p);
   hipEvent_t ev;
   time_begin(c, 0, ev);
   dispatch(p, ct, kmax, [&](auto t_tag, auto v_tag, auto s_tag, auto ct_tag, auto k_tag) {

@@ -305,6 +305,11 @@ bool fused_supported(const Problem& p);
 void fused_propose(Chains& c, bool host_p, int L, int integrator, uint64_t seed, int64_t prop,
                    int randomize, int autotune, double target, double learning_rate,
                    int64_t trace_slot, int64_t hist_slot = -1);
+// several device-RNG proposals per launch (small dense float64 targets without
+// an exchange schedule or kernel timing)
+bool fused_runs_many(const Chains& c);
+void fused_run(Chains& c, int64_t count, int L, int integrator, uint64_t seed, int64_t prop, int randomize,
+               int autotune, double target, double learning_rate, int64_t thinning, int64_t slot0, int64_t hist0);
 void fused_misfit(Chains& c, const void* X, double* out);
 void fused_gradient(Chains& c, const void* X, double* out);
 
