@@ -197,10 +197,12 @@ static void build_sell(Problem& P, Sell& S, int64_t rows, int64_t cols,
   HMC_REQUIRE(cols <= kSellMaxDim && rows <= kSellMaxDim, HMC_ERR_UNSUPPORTED,
               "sparse operator with more than 65472 rows or columns exceeds the fused engine's LDS tile");
   S.nslices = (rows + 63) / 64;
-  // Each lane's entries are stored in groups of kSellGroup consecutive k
-  // (entry k of lane r at base + (k / G) * 64 * G + r * G + k % G), so slice
-  // widths are rounded up to a multiple of the group; padding entries hold
-  // column 0 and value 0.
+  // Each lane's entries are stored in groups of kSellGroup consecutive k, so
+  // slice widths are rounded up to a multiple of the group.  A group's columns
+  // follow each other lane by lane (entry k of lane r at base + (k / G) * 64 * G
+  // + r * G + k % G: 16 bytes a lane); its values are stored as 16-byte pieces,
+  // each of all 64 lanes, so that every load of a wave is 1024 contiguous bytes.
+  // Padding entries hold column 0 and value 0.
   std::vector<int32_t> base(S.nslices), width(S.nslices), perm(S.nslices * 64, -1);
   int64_t total = 0;
   int maxw = 0;
@@ -245,12 +247,17 @@ static void build_sell(Problem& P, Sell& S, int64_t rows, int64_t cols,
     for (int r = 0; r < 64; ++r) {
       const int32_t row = perm[s * 64 + r];
       for (int k = 0; k < width[s]; ++k) {
-        const int64_t o = base[s] + (k / kSellGroup) * 64 * kSellGroup + r * kSellGroup + k % kSellGroup;
+        const int64_t g = base[s] + (k / kSellGroup) * 64 * kSellGroup, e0 = k % kSellGroup;
+        const int64_t o = g + r * kSellGroup + e0;
+        auto slot = [&](int dt) {
+          const int64_t per = 16 / (int64_t)dtype_size(dt);
+          return g + e0 / per * 64 * per + r * per + e0 % per;
+        };
         const int32_t e = seq[r][k];
         if (e >= 0) {
           col[o] = (uint16_t)lane_cols[r][e];
-          store_elem(vtraj.data(), traj_dt, o, val[ptr[row] + e]);
-          if (!alias) store_elem(vtgt.data(), tgt_dt, o, val[ptr[row] + e]);
+          store_elem(vtraj.data(), traj_dt, slot(traj_dt), val[ptr[row] + e]);
+          if (!alias) store_elem(vtgt.data(), tgt_dt, slot(tgt_dt), val[ptr[row] + e]);
         } else {
           const int32_t q = -(e + 1);               // padding: value 0 on a free residue
           col[o] = (uint16_t)(q < cols ? q : 0);

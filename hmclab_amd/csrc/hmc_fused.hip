@@ -52,11 +52,17 @@ template <>
 struct TypeOf<HMC_F32> { using T = float; };
 
 // One SELL row of a lane: acc[c] += sum_k val[k] * in[col[k]][c], k ascending.
-// Slices store each lane's entries in groups of SELL_G consecutive k: entry k
-// of lane r sits at base + (k / SELL_G) * 64 * SELL_G + r * SELL_G + k % SELL_G,
-// and slice widths are multiples of SELL_G, so one group is one 16-byte column
-// load and 16-byte value loads (three vector-memory instructions per 8 entries
-// for float32 values instead of sixteen).  The sum order is k ascending.
+// Slices store each lane's entries in groups of SELL_G consecutive k; slice
+// widths are multiples of SELL_G, so one group is one 16-byte column load and
+// 16-byte value loads (three vector-memory instructions per 8 entries for
+// float32 values instead of sixteen).  Every load of a wave is 1024 contiguous
+// bytes: the columns of a group lie lane by lane, its values in pieces of 16
+// bytes a lane.  A stage is bound by streaming the operator from L2 (64 bytes
+// per clock and CU at most); with a lane's 64 bytes of float64 values together
+// each load touched four times as many cache lines: 41 x 37 cells, 777 rays, 150
+// chains 308 -> 214 us per proposal (five 4-stage steps), 64 x 64, 2000 rays, 100
+// chains 966 -> 604 us (117 GB/s per CU), float32 436 -> 417 us.
+// The sum order is k ascending.
 constexpr int SELL_G = kSellGroup;
 
 // Buffer resource over n bytes of a matrix array (gfx9 raw buffer, stride 0:
@@ -77,7 +83,7 @@ template <typename Acc, typename V>
 __device__ inline void load_group(__amdgpu_buffer_rsrc_t r, int voff, int soff, Acc out[SELL_G]) {
 #pragma unroll
   for (int h = 0; h < SELL_G * (int)sizeof(V) / 16; ++h) {
-    const uint4 q = buf_load16(r, voff + 16 * h, soff);
+    const uint4 q = buf_load16(r, voff + 1024 * h, soff);
     if constexpr (sizeof(V) == 4) {
       const float4 f = __builtin_bit_cast(float4, q);
       out[4 * h] = (Acc)f.x;
@@ -136,7 +142,7 @@ __device__ inline void sell_row(const DevSell& S, const V* __restrict__ valp, in
   if (width <= 0) return;
   const __amdgpu_buffer_rsrc_t rc = sell_rsrc(S.col, S.total * 2);
   const __amdgpu_buffer_rsrc_t rv = sell_rsrc(valp, S.total * (int64_t)sizeof(V));
-  const int vc = lane * SELL_G * 2, vv = lane * SELL_G * (int)sizeof(V);
+  const int vc = lane * SELL_G * 2, vv = lane * 16;
   const uint32_t inb = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)in;
   constexpr int RB = CT * (int)sizeof(Tin);   // bytes of one LDS row
   int sc = (int)base * 2, sv = (int)base * (int)sizeof(V);
@@ -1181,21 +1187,23 @@ static int fused_ct(const Problem& p, int64_t B, size_t& lds_bytes) {
   int maxlds = 65536;
   HMC_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
   const size_t budget = (size_t)maxlds - 2048;
-  // float32 sparse operators prefer 4 chains per workgroup once there are
-  // enough chains for a workgroup per CU: each matrix byte streamed from L2
-  // serves 4 chains (64x64 tomography, 2000 rays, 1024 chains: 0.93 ms per
-  // proposal against 1.34 ms with 2); otherwise, and for dense operators,
-  // 2 chains (half the LDS per workgroup, two workgroups per CU)
+  // As few chains per workgroup as give no CU a second one, since a
+  // workgroup's matrix stream takes about as long for one chain as for more,
+  // and a second round doubles the time.  us per proposal of five 4-stage steps
+  // with 1, 2 and 4 chains per workgroup, float32: 64 x 64 cells, 2000 rays, 100
+  // chains 417, 434, 593; 400 chains 859, 478, 615; 1024 chains 1756, 993, 708;
+  // 41 x 37 cells, 777 rays, 600 chains 445, 336, 236.  float64 with 1 and 2: 41 x
+  // 37, 150 chains 214, 233; 600 chains 634, 471.  Dense operators take 2 beyond one per
+  // CU (400 x 250, float32, L = 10: 100 chains 85, 94, 114; 400 chains 106, 99, 117;
+  // 700 x 800, 100 chains 1378, 1474, 1576; float64 1598, 1693).
   int n_cu = 256;
   HMC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-  const int cands_sparse_f32[] = {4, 2, 1};
-  const int cands_f32[] = {2, 4, 1};
-  const int cands_f64[] = {2, 1};
-  const int* cands = p.state_dtype == HMC_F64 ? cands_f64
-                     : (p.op == 2 && B >= 4 * (int64_t)n_cu) ? cands_sparse_f32 : cands_f32;
-  const int ncand = p.state_dtype == HMC_F64 ? 2 : 3;
-  for (int i = 0; i < ncand; ++i) {
-    const int ct = cands[i];
+  const int most = p.state_dtype == HMC_F64 ? 2 : 4;
+  int cands[3] = {2, 4, 1};
+  if (B <= n_cu) cands[0] = 1, cands[1] = 2, cands[2] = 4;
+  else if (p.op == 2 && B > 2 * (int64_t)n_cu) cands[0] = 4, cands[1] = 2, cands[2] = 1;
+  for (const int ct : cands) {
+    if (ct > most) continue;
     if (p.fused_ct > 0 && ct != p.fused_ct) continue;
     const size_t bytes = (size_t)(round_up(p.d, 2) + round_up(p.n, 2)) * ct * es;
     if (bytes > budget) continue;
@@ -1213,7 +1221,7 @@ static int fused_kmax(const Problem& p) {
   const int nw = fu_nw(p);
   const int64_t per_wave = (nslices + nw - 1) / nw;
   if (per_wave <= 2) return 2;
-  if (nw == 16 && per_wave <= 4) return 4;   // instantiated for the 16-wave (float32 sparse) kernels only
+  if (p.op == 2 && per_wave <= 4) return 4;   // instantiated for the sparse kernels only
   if (per_wave <= 8) return 8;
   if (per_wave <= 16) return 16;
   throw Error{HMC_ERR_UNSUPPORTED, "fused engine supports up to 8192 parameters"};
@@ -1352,7 +1360,7 @@ template <class F>
 static void dispatch(const Problem& p, int ct, int kmax, F&& f) {
   auto by_k = [&](auto t_tag, auto v_tag, auto s_tag, auto ct_tag) {
     using T = typename decltype(t_tag)::type;
-    if constexpr (decltype(s_tag)::value && std::is_same<T, float>::value) {
+    if constexpr (decltype(s_tag)::value) {
       if (kmax == 4) {
         f(t_tag, v_tag, s_tag, ct_tag, std::integral_constant<int, 4>{});
         return;

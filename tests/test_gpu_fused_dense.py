@@ -105,3 +105,33 @@ def test_fused_dense_trace_capacity():
     X, chi = ch.read_trace(0, 3)
     assert np.allclose(X[2], ch.get_state()[0], rtol=0, atol=0)
     p.close()
+
+
+@pytest.mark.parametrize("B", [1, 256, 257, 512, 513])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_fused_tile_rule(B, precision):
+    """The chains per workgroup that the number of chains picks, on a sparse and
+    a dense operator: equal bits with one chain per workgroup."""
+    import scipy.sparse as sp
+    from hmclab_amd._lib import PRIOR_NORMAL
+    from hmclab_amd.engine import Chains, Problem
+
+    n, d = 75, 210
+    rng = np.random.default_rng(B)
+    G = rng.normal(size=(n, d)) / np.sqrt(n) * (rng.uniform(size=(n, d)) < 0.2)
+    x0 = rng.normal(size=(B, d))
+    for setter in (lambda p: p.set_csr(sp.csr_matrix(G), np.ones(n), 0.5), lambda p: p.set_dense(G, np.ones(n), 0.5)):
+        out = []
+        for tiles in (0, 1):
+            p = Problem(d, precision=precision, engine="fused")
+            p.set_option("fused_tile_chains", tiles)
+            setter(p)
+            p.add_prior(PRIOR_NORMAL, np.zeros(d), np.ones(d))
+            ch = Chains(p, B)
+            ch.set_state(x0)
+            step, acc = ch.run(3, 4, 0.2, seed=5)
+            out.append((*ch.get_state(), acc))
+            p.close()
+        assert out[0][2].sum() > 0
+        for a, b in zip(*out):
+            assert np.array_equal(a, b)
