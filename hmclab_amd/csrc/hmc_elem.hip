@@ -376,6 +376,20 @@ void elem_load_rows(Chains& c, const double* src, void* dst, uint16_t* hi, uint1
   HMC_HIP(hipGetLastError());
 }
 
+// One block per row and round; bound by memory (tens of microseconds for a
+// transfer of milliseconds).
+__global__ void k_copy_rows(const double* __restrict__ src, int64_t lds, double* __restrict__ dst, int64_t ldd,
+                            int64_t rows, int64_t d) {
+  for (int64_t r = blockIdx.x; r < rows; r += gridDim.x)
+    for (int64_t j = threadIdx.x; j < d; j += blockDim.x) dst[r * ldd + j] = src[r * lds + j];
+}
+
+void elem_copy_rows(Chains& c, const double* src, int64_t lds, double* dst, int64_t ldd, int64_t rows) {
+  hipLaunchKernelGGL(k_copy_rows, dim3((unsigned)std::min<int64_t>(rows, 4096)), dim3(256), 0, c.p->stream, src, lds,
+                     dst, ldd, rows, c.p->d);
+  HMC_HIP(hipGetLastError());
+}
+
 void elem_store_rows(Chains& c, const void* src, int src_dtype, int64_t ld, double* dst) {
   Problem& p = *c.p;
   const dim3 grid((unsigned)std::min<int64_t>((p.d + 255) / 256, 64), (unsigned)c.B);

@@ -120,6 +120,7 @@ struct Chains {
   void* xt = nullptr;       // trajectory positions
   void* pt = nullptr;       // trajectory momenta
   double* p_host = nullptr; // host-supplied momenta staging [B_pad][ldx] f64
+  double* pack = nullptr;   // the same rows without padding [B][d] (evaluations of padded rows)
   uint16_t* xh = nullptr;   // bf16 hi/lo planes of xt (GEMM engine, BF16)
   uint16_t* xl = nullptr;
   uint16_t* rh = nullptr;   // bf16 hi/lo planes of the residual
@@ -290,6 +291,8 @@ void elem_metropolis(Chains& c, bool have_partials, int autotune, double target,
 void elem_finish_misfit(Chains& c, const void* X, bool have_partials, double* out);
 // convert f64 host-layout rows into state dtype rows (+bf16 planes when given)
 void elem_load_rows(Chains& c, const double* src, void* dst, uint16_t* hi, uint16_t* lo);
+// rows of d doubles between row strides
+void elem_copy_rows(Chains& c, const double* src, int64_t lds, double* dst, int64_t ldd, int64_t rows);
 void elem_store_rows(Chains& c, const void* src, int src_dtype, int64_t ld, double* dst);
 void elem_oob_flags(Chains& c, const void* X);
 // one replica-exchange event over npairs pairs (device array [2*npairs]); u: device
