@@ -227,9 +227,14 @@ __global__ __launch_bounds__(256) void k_set_resid(const SetDesc* __restrict__ d
 // ---------------------------------------------------------------------------
 // residual, LDS-staged variant: the tile's 64*RW rows of G are read KC (64 or
 // 128) columns at a time, KC/4 lanes per row (256 or 512 contiguous bytes per
-// row), into LDS through registers (the next chunk's loads are in flight
-// while the current chunk's MFMAs run); the MFMA sequence per accumulator is
-// the one of k_set_resid (k = 16 s + 4 q + e), so all give identical results.
+// row), into LDS through registers (the next chunk's loads, for 64-row tiles the
+// next two chunks', are in flight while the current chunk's MFMAs run); the MFMA
+// sequence per accumulator is the one of k_set_resid (k = 16 s + 4 q + e), so all
+// give identical results.  What bounds it: a tile's serial chain of chunks (loads,
+// LDS, KC / 4 dependent MFMAs), the longest tiles lasting about half a launch.
+// 96 problems of 50 to 2000 parameters, 90 steps: 54 us a step, with two chunks in
+// flight 50, and with a whole chunk's MFMAs unrolled (their LDS reads run ahead,
+// no branch between them) 46; waits counted exactly per chunk gained nothing more.
 //
 // KICK = 1: the premultiplied step on rows of H instead of G.  H is symmetric,
 // so the tile's rows j give (H x)_j = sum_k H[j][k] x[k] for its 64*RW
@@ -254,6 +259,7 @@ __global__ __launch_bounds__(256) void k_set_resid_lds(const SetDesc* __restrict
   constexpr int LPR = KC / 4, RPP = 256 / LPR;   // loader lanes per row, rows per pass
   constexpr int GPT = ROWS / RPP;                // float4 loads of G per thread per chunk
   constexpr int XPT = SC / RPP;                  // ... of x (KC = 64: 1, 128: 2)
+  constexpr int NS = RW == 1 ? 2 : 1;            // register sets: chunks in flight behind the one in LDS
   static_assert(KC == 64 || KC == 128, "chunk width");
   __shared__ __attribute__((aligned(16))) float Gs[ROWS * LD];
   __shared__ __attribute__((aligned(16))) float Xs[SC * LD];
@@ -271,25 +277,32 @@ __global__ __launch_bounds__(256) void k_set_resid_lds(const SetDesc* __restrict
   const float* Xp = Xin + D.x_off;
   // loader mapping: thread tid covers column 4 * (tid % LPR) of rows tid / LPR + RPP j
   const int lc = 4 * (tid % LPR), lr = tid / LPR;
-  floatx4 gr[GPT], xr[XPT];
-  auto gload = [&](int k0) {
-    const int col = k0 + lc;
+  // Rows past the operator and columns past ldg are read from the last one there
+  // is: the former belong to inactive accumulators, the latter are past kmax.
+  // The loads are unconditional: a condition on each made the wait for a chunk
+  // one for everything behind it.
+  const float* gp[GPT];
+  const float* xp[XPT];
 #pragma unroll
-    for (int j = 0; j < GPT; ++j) {
-      const int row = r0 + lr + RPP * j;
-      gr[j] = (row < nrow && col < D.ldg) ? *(const floatx4*)(Gp + (int64_t)row * D.ldg + col)
-                                           : floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+  for (int j = 0; j < GPT; ++j) {
+    const int row = r0 + lr + RPP * j;
+    gp[j] = Gp + (int64_t)(row < nrow ? row : nrow - 1) * D.ldg;
+  }
 #pragma unroll
-    for (int j = 0; j < XPT; ++j)
-      xr[j] = (col < D.ldg) ? *(const floatx4*)(Xp + (int64_t)(lr + RPP * j) * D.ldg + col)
-                            : floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < XPT; ++j) xp[j] = Xp + (int64_t)(lr + RPP * j) * D.ldg;
+  floatx4 gr[NS][GPT], xr[NS][XPT];
+  auto gload = [&](int u, int k0) __attribute__((always_inline)) {
+    const int col = k0 + lc < D.ldg ? k0 + lc : D.ldg - 4;
+#pragma unroll
+    for (int j = 0; j < GPT; ++j) gr[u][j] = *(const floatx4*)(gp[j] + col);
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) xr[u][j] = *(const floatx4*)(xp[j] + col);
   };
-  auto sstore = [&]() {
+  auto sstore = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < GPT; ++j) *(floatx4*)(&Gs[(lr + RPP * j) * LD + lc]) = gr[j];
+    for (int j = 0; j < GPT; ++j) *(floatx4*)(&Gs[(lr + RPP * j) * LD + lc]) = gr[u][j];
 #pragma unroll
-    for (int j = 0; j < XPT; ++j) *(floatx4*)(&Xs[(lr + RPP * j) * LD + lc]) = xr[j];
+    for (int j = 0; j < XPT; ++j) *(floatx4*)(&Xs[(lr + RPP * j) * LD + lc]) = xr[u][j];
   };
   floatx4 acc[RW];
   bool act[RW];
@@ -298,24 +311,37 @@ __global__ __launch_bounds__(256) void k_set_resid_lds(const SetDesc* __restrict
     acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
     act[r] = r0 + wv * 16 * RW + 16 * r < nr;
   }
-  gload(0);
-  for (int k0 = 0; k0 < D.ldg; k0 += KC) {
+#pragma unroll
+  for (int u = 0; u < NS; ++u) gload(u, u * KC);
+  auto chunk = [&](int u, int k0) __attribute__((always_inline)) {
     __syncthreads();
-    sstore();
+    sstore(u);
     __syncthreads();
-    if (k0 + KC < D.ldg) gload(k0 + KC);
-    const int kmax = D.ldg - k0 < KC ? D.ldg - k0 : KC;   // a multiple of 16
-    for (int s16 = 0; s16 < kmax; s16 += 16) {
+    gload(u, k0 + NS * KC);
+    auto mm = [&](int s16) __attribute__((always_inline)) {
       const floatx4 b = *(const floatx4*)(&Xs[i * LD + s16 + 4 * q]);
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
-        if (!act[r]) continue;
         const floatx4 a = *(const floatx4*)(&Gs[(wv * 16 * RW + 16 * r + i) * LD + s16 + 4 * q]);
         acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], acc[r], 0, 0, 0);
         acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], acc[r], 0, 0, 0);
         acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], acc[r], 0, 0, 0);
         acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], b[3], acc[r], 0, 0, 0);
       }
+    };
+    const int kmax = D.ldg - k0;   // a multiple of 16
+    if (kmax >= KC) {
+#pragma unroll
+      for (int s16 = 0; s16 < KC; s16 += 16) mm(s16);
+    } else {
+      for (int s16 = 0; s16 < kmax; s16 += 16) mm(s16);
+    }
+  };
+  for (int k0 = 0; k0 < D.ldg;) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      if (k0 < D.ldg) chunk(u, k0);
+      k0 += KC;
     }
   }
   if (KICK) {
