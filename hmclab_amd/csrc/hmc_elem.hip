@@ -12,8 +12,9 @@ namespace hmc {
 // Threads of a chain's workgroup: the loops over a chain's parameters are bound
 // by the latency of their loads, one round per EW_NT parameters.  Two proposals of
 // 200 chains of 5000 parameters (bf16 trajectories, everything included): 1595 us
-// with 256, 1557 with 512, 1542 with 1024; 512 chains of 8192: 6397, 6370, 6400
-// (with 1024 the momentum draw's registers allow one workgroup per CU).
+// with 256, 1557 with 512, 1542 with 1024; one of 512 chains of 8192, against the
+// time with 256: 0.995 with 512, 1.00 with 1024 (the momentum draw's registers
+// then allow one workgroup per CU).
 constexpr int EW_NT = 512;
 
 // bf16 planes for the GEMM engine: hi/lo of v, or (anchored, l null) one
